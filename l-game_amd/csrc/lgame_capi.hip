@@ -121,6 +121,12 @@ __global__ void k_to_float(float *dst, const double *src, size_t n) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) dst[i] = (float)src[i];
 }
 
+// dst += src (the two parts of a checkpoint's pressure gradient)
+template <class T>
+__global__ void k_add_to(T *dst, const T *src, size_t n) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) dst[i] = dst[i] + src[i];
+}
+
 // Klemp damping prefactor at w levels, 1 + damping_coeff*dtime (mo_column_solvers.F90:190-196)
 double klemp_prefactor(const lgame_cfg &cf, double z) {
   const double start = cf.klemp_begin_rel * cf.toa;
@@ -365,8 +371,7 @@ int enqueue_pchevi(const CtxT<R> &c, const StateDev &old, const StateDev &nw, in
       LG_LAUNCH_ZFAST(KI_DIFF_MOM, k_diff_mom, nx, ny, nl, c, old);
     }
     if (rk == 1 && c.C.lpbl) LG_LAUNCH(KI_DIFF_DUAL, k_pbl_wind, nx, ny, 1, c, old);
-    if (rk == 1 && (c.C.lklemp || c.C.lmom_h || c.C.lmom_v || c.C.lpbl))
-      LG_LAUNCH(KI_DISSIPATION, k_dissipation, nx, ny, nl, c, old);
+    if (rk == 1 && diss_levels(c) > 0) LG_LAUNCH(KI_DISSIPATION, k_dissipation, nx, ny, diss_levels(c), c, old);
     // the first substep's pressure gradient (manage_p_grad) and, from its values, the wind update;
     // no kernel in between reads or writes what the pressure gradient uses or forms
     if (rk == 1)
@@ -712,7 +717,7 @@ int lgame_init(const lgame_dims *dims, const lgame_cfg *cfg, const lgame_grid_vi
   const size_t fs = (size_t)G.fsize;
   const size_t nstate = (size_t)2 * (nc + 6 + (C.lsoil ? 1 : 0));
   const size_t ndiff = diffusion ? (size_t)14 + nc + 3 * (nc + 1) : 0;  // the diffusion and surface fields of WorkT
-  const size_t nwork = (size_t)nc + 4 + 8 + 6 + 4 + 7 + 10 + 2 + ndiff;
+  const size_t nwork = (size_t)nc + 4 + 5 + 6 + 4 + 7 + 10 + 2 + ndiff;
   const size_t ncol = 13;  // 12 column-scratch fields and the cloud-water sink velocity
   const size_t wbytes = mixed ? sizeof(float) : sizeof(double);
   h->slab_bytes = (nstate + NGRID + ncol) * fs * sizeof(double) + nwork * fs * wbytes + (mixed ? NGRID * fs * sizeof(float) : 0);
@@ -758,14 +763,11 @@ int lgame_init(const lgame_dims *dims, const lgame_cfg *cfg, const lgame_grid_vi
     W.tend_u = take();
     W.tend_v = take();
     W.tend_w = take();
-    W.pnl_u = take();
-    W.pnl_v = take();
-    W.pnl_w = take();
-    W.pl_u = take();
-    W.pl_v = take();
-    W.pl_w = take();
-    W.pold_u = take();
-    W.pold_v = take();
+    W.pg_u = take();
+    W.pg_v = take();
+    W.ps_u = take();
+    W.ps_v = take();
+    W.ps_w = take();
     W.vsg_x = take();
     W.vsg_y = take();
     W.vsg_z = take();
@@ -834,6 +836,7 @@ int lgame_init(const lgame_dims *dims, const lgame_cfg *cfg, const lgame_grid_vi
   }
   e = hipMemsetAsync(h->slab, 0, h->slab_bytes, h->stream);
   h->staging_elems = (size_t)d.ny * d.nx * d.n_layers * (nc > 6 ? nc : 6) + (size_t)(d.ny + 1) * (d.nx + 1) * (d.n_layers + 1);
+  if (h->staging_elems < fs) h->staging_elems = fs;  // a whole box (lgame_checkpoint_load)
   if (e == hipSuccess) e = hipMalloc(&h->staging, h->staging_elems * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&h->red, (size_t)2 * NRED * RED_GRID * sizeof(double) + NRED * sizeof(double));
   if (e == hipSuccess) e = hipMalloc(&h->counter, 2 * sizeof(unsigned long long));
@@ -1187,9 +1190,15 @@ namespace {
 // the surface physics the TKE, viscosity, momentum-diffusion tendencies, heating and
 // mass-diffusion tendencies and the surface turbulence quantities; then the radiation's surface
 // fluxes.
+//
+// The layout gives the pressure gradient eight boxes, of which the first five hold its nonlinear
+// parts at the u, v and w points and the linear ones at u and v: only their sums at u and v are
+// carried, so a save writes the sum as the nonlinear part and zeros for the rest, and a load adds the
+// linear part to the nonlinear one.
 struct Carried {
-  void *p;
+  void *p;  // null: a box that is written as zeros and not read
   size_t bytes;
+  bool add = false;  // written as zeros; on load its values are added to the field p
 };
 
 std::vector<Carried> carried_fields(lgame_handle *h) {
@@ -1197,8 +1206,13 @@ std::vector<Carried> carried_fields(lgame_handle *h) {
   const size_t es = h->mixed ? sizeof(float) : sizeof(double);
   const size_t box = (size_t)h->c.G.fsize * es, lvl = (size_t)h->c.G.lvl * es;
   auto add_work = [&](const auto &w) {
-    for (auto f : {w.pnl_u, w.pnl_v, w.pnl_w, w.pl_u, w.pl_v, w.pl_w, w.pold_u, w.pold_v, w.vsg_x, w.vsg_y, w.vsg_z, w.pvt_x,
-                   w.pvt_y, w.pvt_z, w.u_ph, w.v_ph, w.w_ph, w.v_squared, w.csh, w.heating_diss, w.radiation_tendency, w.tke,
+    v.push_back({(void *)w.pg_u.p, box});
+    v.push_back({(void *)w.pg_v.p, box});
+    v.push_back({nullptr, box});
+    v.push_back({(void *)w.pg_u.p, box, true});
+    v.push_back({(void *)w.pg_v.p, box, true});
+    for (int q = 0; q < 3; ++q) v.push_back({nullptr, box});
+    for (auto f : {w.vsg_x, w.vsg_y, w.vsg_z, w.pvt_x, w.pvt_y, w.pvt_z, w.u_ph, w.v_ph, w.w_ph, w.v_squared, w.csh, w.heating_diss, w.radiation_tendency, w.tke,
                    w.visc, w.mom_x, w.mom_y, w.mom_z, w.tdh})
       if (f.p) v.push_back({(void *)f.p, box});
     for (int jc = 0; jc < h->dims.n_constituents; ++jc)
@@ -1268,7 +1282,10 @@ int lgame_checkpoint_save(lgame_handle *h, void *buf, long long bytes) {
   out += sizeof hd;
   HIPCHK(h, hipStreamSynchronize(h->stream));
   for (auto &f : carried_fields(h)) {
-    HIPCHK(h, hipMemcpy(out, f.p, f.bytes, hipMemcpyDeviceToHost));
+    if (!f.p || f.add)
+      std::memset(out, 0, f.bytes);
+    else
+      HIPCHK(h, hipMemcpy(out, f.p, f.bytes, hipMemcpyDeviceToHost));
     out += f.bytes;
   }
   return LGAME_OK;
@@ -1288,9 +1305,25 @@ int lgame_checkpoint_load(lgame_handle *h, const void *buf, long long bytes) {
   const char *in = (const char *)buf + sizeof hd;
   HIPCHK(h, hipStreamSynchronize(h->stream));
   for (auto &f : carried_fields(h)) {
-    HIPCHK(h, hipMemcpy(f.p, in, f.bytes, hipMemcpyHostToDevice));
+    if (f.add) {  // one box fits the staging buffer
+      HIPCHK(h, hipMemcpy(h->staging, in, f.bytes, hipMemcpyHostToDevice));
+      if (h->mixed)
+        hipLaunchKernelGGL(k_add_to<float>, dim3(1024), dim3(256), 0, h->stream, (float *)f.p, (const float *)h->staging, f.bytes / 4);
+      else
+        hipLaunchKernelGGL(k_add_to<double>, dim3(1024), dim3(256), 0, h->stream, (double *)f.p, (const double *)h->staging, f.bytes / 8);
+      HIPCHK(h, hipGetLastError());
+      HIPCHK(h, hipStreamSynchronize(h->stream));
+    } else if (f.p) {
+      HIPCHK(h, hipMemcpy(f.p, in, f.bytes, hipMemcpyHostToDevice));
+    }
     in += f.bytes;
   }
+  // the dissipation rate is formed (and read) in its levels only
+  auto zero_below = [&](const auto &c) {
+    const size_t es = sizeof(*c.w.heating_diss.p), n = (size_t)diss_levels(c) * (size_t)c.G.lvl;
+    return hipMemset((char *)c.w.heating_diss.p + n * es, 0, ((size_t)c.G.fsize - n) * es);
+  };
+  if (h->c.C.lklemp) HIPCHK(h, h->mixed ? zero_below(h->cf) : zero_below(h->c));
   h->rad_calls = hd.rad_calls;
   return LGAME_OK;
 }

@@ -99,7 +99,10 @@ template <class R>
 struct WorkT {
   Fld<R> tend_rho[MAX_CONST];
   Fld<R> tend_rhotheta_v, tend_u, tend_v, tend_w;
-  Fld<R> pnl_u, pnl_v, pnl_w, pl_u, pl_v, pl_w, pold_u, pold_v;
+  // pressure gradient of the first substep: pg_u, pg_v its nonlinear plus linear part (carried: the
+  // negative is the next step's old gradient); ps_u, ps_v, ps_w its part of the wind tendencies,
+  // old_hor*(old gradient) - cur_hor*pg and -cur_ver*pg, which both substeps start from
+  Fld<R> pg_u, pg_v, ps_u, ps_v, ps_w;
   Fld<R> vsg_x, vsg_y, vsg_z, pvt_x, pvt_y, pvt_z;
   Fld<R> heating_diss, csh, temperature, radiation_tendency;
   Fld<R> eta_x, eta_y, eta_z, u_ph, v_ph, w_ph, v_squared;

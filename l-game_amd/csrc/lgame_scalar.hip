@@ -172,7 +172,7 @@ struct CellIn {
   R told[TR ? 7 : 1], md[TR ? 7 : 1];
 };
 
-template <class R, bool TR, bool DIFF>
+template <class R, bool TR, bool DIFF, bool TOLD>
 __device__ __forceinline__ void load_cell(const CtxT<R> &c, const StateDev &ss, const Lane &p, int jl, CellIn<R, TR> &f) {
   using K = Cons<TR>;
   const Geom &G = c.G;
@@ -180,7 +180,11 @@ __device__ __forceinline__ void load_cell(const CtxT<R> &c, const StateDev &ss, 
   f.az_u = c.g.area_z[i];
   f.az_l = c.g.area_z[i + (ix_t)G.lvl];
   f.V = c.g.volume[i];
-  f.heat = c.w.heating_diss[i] + c.w.radiation_tendency[i] + c.w.csh[i];
+  // heating_diss holds zeros below diss_levels, or where no dissipation is formed what a checkpoint
+  // brought; a dry step has no sediment heating
+  const bool diss = jl <= diss_levels(c) || !c.C.lklemp;
+  f.heat = (diss ? c.w.heating_diss[i] : R(0.0)) + c.w.radiation_tendency[i];
+  if (TR) f.heat = f.heat + c.w.csh[i];
   if (DIFF && c.C.ltemp_h) f.heat = f.heat + c.w.tdh[i];  // diag%temp_diff_heating (of this step's first substep)
   f.temperature = c.w.temperature[i];
   f.exner = c.g.exner_bg[i] + R(ss.exner_pert[i]);
@@ -193,15 +197,15 @@ __device__ __forceinline__ void load_cell(const CtxT<R> &c, const StateDev &ss, 
 #pragma unroll
   for (int q = 0; q < K::nc; ++q) {
     if (!K::tracer(q)) continue;
-    f.told[q] = c.w.tend_rho[q][i];
     f.md[q] = DIFF && c.C.lmass_h ? c.w.mdt[q][i] : R(0.0);
+    f.told[q] = TOLD ? c.w.tend_rho[q][i] : R(0.0);
   }
 }
 
 // the tendencies of cell (ji, jk, jl) from its prepared layer L, its inputs f, the corrections of
 // its upper (L.I) and lower (Ilo) interface and the tracer densities of the layers above and below
-template <class R, bool TR, bool DIFF>
-__device__ __forceinline__ void finish_cell(const CtxT<R> &c, const StateDev &nw, int rk, const Lane &p, int jl,
+template <class R, bool TR, bool DIFF, bool TOLD>
+__device__ __forceinline__ void finish_cell(const CtxT<R> &c, const StateDev &nw, const Lane &p, int jl,
                                             const Prep<R, TR> &L, const CellIn<R, TR> &f, const Corr<R> &Ilo, const R *r_up,
                                             const R *r_lo) {
   using K = Cons<TR>;
@@ -235,7 +239,7 @@ __device__ __forceinline__ void finish_cell(const CtxT<R> &c, const StateDev &nw
   }
   R tt[TR ? 7 : 1];
   if (TR) {
-    const R new_w = rk == 2 ? R(0.5) : R(1.0), old_w = R(1.0) - new_w;
+    const R half = R(0.5);
     const R cu = (jl == nl || jl > nflat) && jl != nflat ? cu_w : R(0.0);
     const R cl = jl == nflat || (jl > nflat && jl != nl) ? cl_w : R(0.0);
 #pragma unroll
@@ -254,7 +258,7 @@ __device__ __forceinline__ void finish_cell(const CtxT<R> &c, const StateDev &nw
       }
       const R d = (L.ht[q] + comp_v) / V;
       const R x = DIFF && c.C.lmass_h ? -d + f.md[q] : -d;
-      tt[q] = old_w * f.told[q] + new_w * x;
+      tt[q] = TOLD ? half * f.told[q] + half * x : x;
     }
   }
   if (!p.cell) return;
@@ -271,8 +275,8 @@ __device__ __forceinline__ void finish_cell(const CtxT<R> &c, const StateDev &nw
 // Launch: a 1-D grid of ceil(nx/62) x ceil(ny/by) x nseg blocks of 64 x by threads (by rows of
 // 64 lanes), dealt to the XCDs so that each takes a contiguous range of tiles with x fastest:
 // the rows above and below a tile are read by the blocks next to it on the same XCD.
-template <class R, bool TR, bool O3, bool DIFF>
-__device__ __forceinline__ void b_scalar_col(const CtxT<R> &c, const StateDev &ss, const StateDev &nw, int rk, int nseg, const Bid bid) {
+template <class R, bool TR, bool O3, bool DIFF, bool TOLD>
+__device__ __forceinline__ void b_scalar_col(const CtxT<R> &c, const StateDev &ss, const StateDev &nw, int nseg, const Bid bid) {
   const Geom &G = c.G;
   const int nx = G.nx, ny = G.ny, nl = G.nl;
   const int tx_n = (nx + SCOL_CELLS - 1) / SCOL_CELLS, ty_n = (ny + (int)blockDim.y - 1) / (int)blockDim.y;
@@ -309,9 +313,9 @@ __device__ __forceinline__ void b_scalar_col(const CtxT<R> &c, const StateDev &s
   for (int jl = l0; jl <= l1; ++jl) {
     // the next layer (at jl = n_layers the padding level n_layers+1, whose values are not used)
     CellIn<R, TR> f;
-    load_cell<R, TR, DIFF>(c, ss, p, jl, f);
+    load_cell<R, TR, DIFF, TOLD>(c, ss, p, jl, f);
     prep_layer<R, TR, O3>(c, ss, nw, p, jl + 1, cur.P, nxt);
-    finish_cell<R, TR, DIFF>(c, nw, rk, p, jl, cur, f, nxt.I, r_up, nxt.r);
+    finish_cell<R, TR, DIFF, TOLD>(c, nw, p, jl, cur, f, nxt.I, r_up, nxt.r);
 #pragma unroll
     for (int qq = 0; qq < (TR ? 7 : 1); ++qq) r_up[qq] = cur.r[qq];
     cur = nxt;
@@ -326,29 +330,36 @@ template <class R>
 __host__ __device__ constexpr bool scol_diff_variant(bool diff) {
   return diff || sizeof(R) == 4;
 }
-template <class R, bool TR, bool O3, bool DIFF>
-__global__ void __launch_bounds__(BX * 4)
-    k_scalar_col(const CtxT<R> c, const StateDev ss, const StateDev nw, int rk, int nseg) {
-  b_scalar_col<R, TR, O3, DIFF>(c, ss, nw, rk, nseg, bid_here());
+// TOLD: the moist second substep, which takes the mean with the first one's tracer tendencies.  The
+// first substep does not read the tendencies of the step before, whose weight is 0 (six fields: 1264
+// -> 1116 us at 512x512x60 in FP64); the two are instantiations of their own because a run-time
+// check of the substep around the loads made the second one 7% slower.
+template <class R, bool TR, bool O3, bool DIFF, bool TOLD>
+__global__ void __launch_bounds__(BX * 4) k_scalar_col(const CtxT<R> c, const StateDev ss, const StateDev nw, int nseg) {
+  b_scalar_col<R, TR, O3, DIFF, TOLD>(c, ss, nw, nseg, bid_here());
 }
+
+// the instantiation for tr (moist), o3, diff and told
+#define LG_SCOL_O3(TR, TOLD)                   \
+  do {                                         \
+    if (o3 && diff) LG_SCOL(TR, true, true, TOLD);        \
+    else if (o3) LG_SCOL(TR, true, false, TOLD);          \
+    else if (diff) LG_SCOL(TR, false, true, TOLD);        \
+    else LG_SCOL(TR, false, false, TOLD);                 \
+  } while (0)
+#define LG_SCOL_DISPATCH                       \
+  if (told) LG_SCOL_O3(true, true);            \
+  else if (tr) LG_SCOL_O3(true, false);        \
+  else LG_SCOL_O3(false, false);
 
 template <class R>
 void launch_scalar_col(const CtxT<R> &c, const StateDev &ss, const StateDev &nw, int rk, int rows, int nseg, hipStream_t st) {
   const int tx_n = (c.G.nx + SCOL_CELLS - 1) / SCOL_CELLS, ty_n = (c.G.ny + rows - 1) / rows;
   const dim3 blk(BX, rows, 1), grd((unsigned)(tx_n * ty_n * nseg));
   const bool tr = c.G.nc > 1, o3 = c.C.order == 3, diff = scol_diff_variant<R>(c.C.ltemp_h || c.C.lmass_h);
-#define LG_SCOL(TR, O3, DIFF) hipLaunchKernelGGL((k_scalar_col<R, TR, O3, DIFF>), grd, blk, 0, st, c, ss, nw, rk, nseg)
-  if (diff) {
-    if (tr && o3) LG_SCOL(true, true, true);
-    else if (tr) LG_SCOL(true, false, true);
-    else if (o3) LG_SCOL(false, true, true);
-    else LG_SCOL(false, false, true);
-  } else {
-    if (tr && o3) LG_SCOL(true, true, false);
-    else if (tr) LG_SCOL(true, false, false);
-    else if (o3) LG_SCOL(false, true, false);
-    else LG_SCOL(false, false, false);
-  }
+const bool told = tr && rk == 2;
+#define LG_SCOL(TR, O3, DIFF, TOLD) hipLaunchKernelGGL((k_scalar_col<R, TR, O3, DIFF, TOLD>), grd, blk, 0, st, c, ss, nw, nseg)
+  LG_SCOL_DISPATCH
 #undef LG_SCOL
 }
 
@@ -356,30 +367,21 @@ template void launch_scalar_col<double>(const CtxT<double> &, const StateDev &, 
 template void launch_scalar_col<float>(const CtxT<float> &, const StateDev &, const StateDev &, int, int, int, hipStream_t);
 
 // ---- the same kernel over a group of domains (one launch) --------------------------------------
-template <class R, bool TR, bool O3, bool DIFF>
+template <class R, bool TR, bool O3, bool DIFF, bool TOLD>
 __global__ void __launch_bounds__(BX * 4)
     kb_scalar_col(const MemberDev<R> *__restrict__ M, const int *__restrict__ prefix, int nm, const BatchArgs a) {
   Bid bid;
   const MemberDev<R> &d = batch_block(M, prefix, nm, PH_SCALAR, bid);
-  b_scalar_col<R, TR, O3, DIFF>(d.c, d.s[a.state_slot], d.s[a.new_slot], a.rk, d.seg, bid);
+  b_scalar_col<R, TR, O3, DIFF, TOLD>(d.c, d.s[a.state_slot], d.s[a.new_slot], d.seg, bid);
 }
 
 template <class R>
 void batch_launch_scalar(dim3 g, dim3 b, hipStream_t st, const MemberDev<R> *M, const int *prefix, int nm, const BatchArgs &a,
                          bool tr, bool o3, bool diff) {
   diff = scol_diff_variant<R>(diff);
-#define LG_SCOL(TR, O3, DIFF) hipLaunchKernelGGL((kb_scalar_col<R, TR, O3, DIFF>), g, b, 0, st, M, prefix, nm, a)
-  if (diff) {
-    if (tr && o3) LG_SCOL(true, true, true);
-    else if (tr) LG_SCOL(true, false, true);
-    else if (o3) LG_SCOL(false, true, true);
-    else LG_SCOL(false, false, true);
-  } else {
-    if (tr && o3) LG_SCOL(true, true, false);
-    else if (tr) LG_SCOL(true, false, false);
-    else if (o3) LG_SCOL(false, true, false);
-    else LG_SCOL(false, false, false);
-  }
+const bool told = tr && a.rk == 2;
+#define LG_SCOL(TR, O3, DIFF, TOLD) hipLaunchKernelGGL((kb_scalar_col<R, TR, O3, DIFF, TOLD>), g, b, 0, st, M, prefix, nm, a)
+  LG_SCOL_DISPATCH
 #undef LG_SCOL
 }
 template void batch_launch_scalar<double>(dim3, dim3, hipStream_t, const MemberDev<double> *, const int *, int, const BatchArgs &,

@@ -93,6 +93,17 @@ __host__ __device__ inline int col_waves(const Geom &G) { return col_waves_per_r
 constexpr int NTR = 6;         // tracers per moist column
 constexpr int GEN_GROUPS = 2;  // 64-column groups per block
 
+// Levels 1..diss_levels in which k_dissipation forms the dissipation rate: with a friction of the wind
+// all of them, with the Klemp layer alone those whose upper or lower interface lies in it (below it
+// every term has a zero factor, the array keeps its initial zeros and is not read), else none.  At
+// 512x512x60 with 24 levels in the layer the FP64 launch takes 115 instead of 249 us.
+template <class R>
+__host__ __device__ inline int diss_levels(const CtxT<R> &c) {
+  if (c.C.lmom_h || c.C.lmom_v || c.C.lpbl) return c.G.nl;
+  if (!c.C.lklemp) return 0;
+  return c.C.n_damping_levels < c.G.nl ? c.C.n_damping_levels : c.G.nl;
+}
+
 // Optional timing hook around kernel groups (0 = vertical solver, 1 = tracer solver, 2 = step,
 // 3 = radiation; PROF_KERNEL0 + KernelId for every stencil kernel when `kernels` is set).
 constexpr int PROF_KERNEL0 = 8;

@@ -120,6 +120,26 @@ __global__ void __launch_bounds__(BX * BY) k_theta_edge(const CtxT<R> c, const S
   b_theta_edge(c, s, nfield, bid_here());
 }
 
+// the weights of a substep's tendency update
+template <class R>
+struct VtWeights {
+  R new_w, old_w, cur_hor, old_hor, cur_ver;
+  bool mom;    // diag%mom_diff_tend_* are added (zero arrays otherwise)
+  bool first;  // the first substep, whose old_w is 0: the previous step's tendency is not read
+};
+template <class R>
+__device__ __forceinline__ VtWeights<R> vt_weights(const CtxT<R> &c, int rk) {
+  VtWeights<R> w;
+  w.new_w = rk == 2 ? R(0.5) : R(1.0);
+  w.old_w = R(1.0) - w.new_w;
+  w.cur_hor = R(0.5) + R(IMPL_THERMO_WEIGHT);
+  w.old_hor = R(1.0) - w.cur_hor;
+  w.cur_ver = R(1.0) - R(IMPL_THERMO_WEIGHT);
+  w.mom = c.C.lmom_h || c.C.lmom_v || c.C.lpbl;
+  w.first = rk == 1;
+  return w;
+}
+
 // ---------------------------------------------------------------------------------------------
 // manage_p_grad, mo_p_grad.F90:20-104 (luse_bg_state): nonlinear and linear pressure gradient
 // accelerations at u, v and w points, scaled by the condensate deceleration factor.
@@ -127,17 +147,19 @@ __global__ void __launch_bounds__(BX * BY) k_theta_edge(const CtxT<R> c, const S
 // The pressure-gradient accelerations at the u, v and w points of one cell (ji <= ny, jk <= nx). Its west, south and upper neighbours and the cell itself are shared by the three
 // points, so every state value, metric and deceleration factor is loaded or computed once and
 // then combined with the expressions of grad_hor_x/_y, remap_ver2hor_x/_y and the w-point
-// gradient, in their order.  Returns the values it stores at the cell's three points.
+// gradient, in their order.
+// The parts enter the wind tendencies only as old_hor*pold - cur_hor*(pnl + pl) (u, v) and
+// -cur_ver*(pnl + pl) (w), and the next step reads them only as pold = -pnl - pl = -(pnl + pl): so
+// the sum and the weighted sum are stored, not the parts and pold (the same bits; 11 loads and stores
+// of a field less per step and point).  Returns the weighted sums.
 template <class R>
 struct PGrad {
-  R nl_u, l_u, old_u;  // u point: nonlinear and linear parts, and the previous step's sum (pold)
-  R nl_v, l_v, old_v;  // v point
-  R nl_w, l_w;         // w point (levels 2..n_layers)
+  R u, v, w;  // its part of the wind tendency at the u, v and w point (w at levels 2..n_layers)
 };
 template <class R>
-__device__ __forceinline__ PGrad<R> pgrad_interior(const CtxT<R> &c, const StateDev &s, int lfirst, int ji, int jk, int jl) {
+__device__ __forceinline__ PGrad<R> pgrad_interior(const CtxT<R> &c, const StateDev &s, const VtWeights<R> &wt, int lfirst, int ji, int jk, int jl) {
   PGrad<R> o;
-  o.nl_w = o.l_w = R(0.0);
+  o.w = R(0.0);
   const int nx = c.G.nx, ny = c.G.ny, nl = c.G.nl, nlev = c.G.nlev, nflat = c.G.nflat;
   const bool o3 = c.C.order == 3;
   const Geom &G = c.G;
@@ -173,11 +195,8 @@ __device__ __forceinline__ PGrad<R> pgrad_interior(const CtxT<R> &c, const State
   const R tpC = R(tp[iC]), thC = c.g.theta_v_bg[iC] + tpC, dC = decel_at(iC);
   // u point
   {
-    R pold = R(0.0);
-    if (!lfirst) {
-      pold = -c.w.pnl_u[iC] - R(1.0) * c.w.pl_u[iC];
-      c.w.pold_u[iC] = pold;
-    }
+    R pg_old = R(0.0);
+    if (!lfirst) pg_old = c.w.pg_u[iC];
     R g = (eC - eW) / c.g.dx[iC];
     if (terr) {
       R r = R(0.0);
@@ -199,30 +218,20 @@ __device__ __forceinline__ PGrad<R> pgrad_interior(const CtxT<R> &c, const State
       lu = R(0.5) * (tpW + tpC) * c.g.ebg_u[iC];
     }
     const R d = R(0.5) * (decel_at(iW) + dC);
-    const R nlu = d * t, llu = d * lu;
-    c.w.pnl_u[iC] = nlu;
-    c.w.pl_u[iC] = llu;
-    if (lfirst) {
-      pold = -nlu - R(1.0) * llu;
-      c.w.pold_u[iC] = pold;
-    }
-    o.nl_u = nlu;
-    o.l_u = llu;
-    o.old_u = pold;
+    const R pg = d * t + d * lu;
+    o.u = wt.old_hor * -(lfirst ? pg : pg_old) - wt.cur_hor * pg;
+    c.w.pg_u[iC] = pg;
+    c.w.ps_u[iC] = o.u;
     if (jk == 1) {  // column nx+1 is the copy of column 1
       const ix_t iX = LG_IX(G, ji, nx + 1, jl);
-      c.w.pnl_u[iX] = nlu;
-      c.w.pl_u[iX] = llu;
-      c.w.pold_u[iX] = pold;
+      c.w.pg_u[iX] = pg;
+      c.w.ps_u[iX] = o.u;
     }
   }
   // v point
   {
-    R pold = R(0.0);
-    if (!lfirst) {
-      pold = -c.w.pnl_v[iC] - R(1.0) * c.w.pl_v[iC];
-      c.w.pold_v[iC] = pold;
-    }
+    R pg_old = R(0.0);
+    if (!lfirst) pg_old = c.w.pg_v[iC];
     R g = (eS - eC) / c.g.dy[iC];
     if (terr) {
       R r = R(0.0);
@@ -244,21 +253,14 @@ __device__ __forceinline__ PGrad<R> pgrad_interior(const CtxT<R> &c, const State
       lv = R(0.5) * (tpS + tpC) * c.g.ebg_v[iC];
     }
     const R d = R(0.5) * (decel_at(iS) + dC);
-    const R nlv = d * t, llv = d * lv;
-    c.w.pnl_v[iC] = nlv;
-    c.w.pl_v[iC] = llv;
-    if (lfirst) {
-      pold = -nlv - R(1.0) * llv;
-      c.w.pold_v[iC] = pold;
-    }
-    o.nl_v = nlv;
-    o.l_v = llv;
-    o.old_v = pold;
+    const R pg = d * t + d * lv;
+    o.v = wt.old_hor * -(lfirst ? pg : pg_old) - wt.cur_hor * pg;
+    c.w.pg_v[iC] = pg;
+    c.w.ps_v[iC] = o.v;
     if (ji == 1) {  // row ny+1 is the copy of row 1
       const ix_t iY = LG_IX(G, ny + 1, jk, jl);
-      c.w.pnl_v[iY] = nlv;
-      c.w.pl_v[iY] = llv;
-      c.w.pold_v[iY] = pold;
+      c.w.pg_v[iY] = pg;
+      c.w.ps_v[iY] = o.v;
     }
   }
   // w point, levels 2..n_layers
@@ -268,10 +270,8 @@ __device__ __forceinline__ PGrad<R> pgrad_interior(const CtxT<R> &c, const State
     const R t = R(0.5) * ((c.g.theta_v_bg[iA] + tpA) + thC) * vC;
     const R lw = R(0.5) * (tpA + tpC) * c.g.ebg_w[iC];
     const R d = R(0.5) * (decel_at(iA) + dC);
-    o.nl_w = d * t;
-    o.l_w = d * lw;
-    c.w.pnl_w[iC] = o.nl_w;
-    c.w.pl_w[iC] = o.l_w;
+    o.w = -wt.cur_ver * (d * t + d * lw);
+    c.w.ps_w[iC] = o.w;
   }
   return o;
 }
@@ -643,7 +643,7 @@ __device__ __forceinline__ void b_dissipation(const CtxT<R> &c, const StateDev &
   KIDX;
   const Geom &G = c.G;
   const int nl = G.nl;
-  if (jk > G.nx || ji > G.ny || jl > nl) return;
+  if (jk > G.nx || ji > G.ny || jl > diss_levels(c)) return;
   const ix_t i = LG_IX(G, ji, jk, jl), ib = LG_IX(G, ji, jk, jl + 1);
   R mz0 = R(0.0), mz1 = R(0.0);
   if (c.C.lmom_v) {
@@ -698,48 +698,35 @@ __global__ void __launch_bounds__(BX * BY) k_dissipation(const CtxT<R> c, const 
 // explicit wind tendencies (mo_vector_tend_expl.F90:128-180) and the forward update of u, v
 // (mo_manage_pchevi.F90:86-89)
 // ---------------------------------------------------------------------------------------------
-// the weights of a substep's tendency update
+// the tendency at one point: the first substep takes x, the second the weighted mean with the first's
 template <class R>
-struct VtWeights {
-  R new_w, old_w, cur_hor, old_hor, cur_ver;
-  bool mom;  // diag%mom_diff_tend_* are added (zero arrays otherwise)
-};
-template <class R>
-__device__ __forceinline__ VtWeights<R> vt_weights(const CtxT<R> &c, int rk) {
-  VtWeights<R> w;
-  w.new_w = rk == 2 ? R(0.5) : R(1.0);
-  w.old_w = R(1.0) - w.new_w;
-  w.cur_hor = R(0.5) + R(IMPL_THERMO_WEIGHT);
-  w.old_hor = R(1.0) - w.cur_hor;
-  w.cur_ver = R(1.0) - R(IMPL_THERMO_WEIGHT);
-  w.mom = c.C.lmom_h || c.C.lmom_v || c.C.lpbl;
-  return w;
+__device__ __forceinline__ R vt_mean(const VtWeights<R> &w, Fld<const R> tend, ix_t i, R x) {
+  return w.first ? x : w.old_w * tend[i] + w.new_w * x;
 }
-// the u point at index i, from its pressure-gradient terms (pold, pnl, pl)
-// and the kinetic-energy gradient and vorticity flux term there (vsg, pvt)
+// the u point at index i, from its pressure-gradient part ps and the kinetic-energy gradient and
+// vorticity flux term there (vsg, pvt)
 template <class R>
-__device__ __forceinline__ void vt_u(const CtxT<R> &c, const StateDev &old, const StateDev &nw, const VtWeights<R> &w, ix_t i,
-                                     R pold, R pnl, R pl, R vsg, R pvt) {
-  R x = w.old_hor * pold - w.cur_hor * (pnl + pl) - R(0.5) * vsg + pvt;
+__device__ __forceinline__ void vt_u(const CtxT<R> &c, const StateDev &old, const StateDev &nw, const VtWeights<R> &w, ix_t i, R ps,
+                                     R vsg, R pvt) {
+  R x = ps - R(0.5) * vsg + pvt;
   if (w.mom) x = x + c.w.mom_x[i];
-  const R t = w.old_w * c.w.tend_u[i] + w.new_w * x;
+  const R t = vt_mean<R>(w, c.w.tend_u, i, x);
   c.w.tend_u[i] = t;
   nw.wind_u[i] = old.wind_u[i] + c.C.dtime * (double)t;  // FP64 state update
 }
 template <class R>
-__device__ __forceinline__ void vt_v(const CtxT<R> &c, const StateDev &old, const StateDev &nw, const VtWeights<R> &w, ix_t i,
-                                     R pold, R pnl, R pl, R vsg, R pvt) {
-  R x = w.old_hor * pold - w.cur_hor * (pnl + pl) - R(0.5) * vsg + pvt;
+__device__ __forceinline__ void vt_v(const CtxT<R> &c, const StateDev &old, const StateDev &nw, const VtWeights<R> &w, ix_t i, R ps,
+                                     R vsg, R pvt) {
+  R x = ps - R(0.5) * vsg + pvt;
   if (w.mom) x = x + c.w.mom_y[i];
-  const R t = w.old_w * c.w.tend_v[i] + w.new_w * x;
+  const R t = vt_mean<R>(w, c.w.tend_v, i, x);
   c.w.tend_v[i] = t;
   nw.wind_v[i] = old.wind_v[i] + c.C.dtime * (double)t;
 }
 // the w point of cell (ji, jk, jl), jl >= 2
 template <class R>
-__device__ __forceinline__ void vt_w(const CtxT<R> &c, const VtWeights<R> &w, int ji, int jk, int jl, ix_t i, R pnl, R pl, R vsg,
-                                     R pvt) {
-  R x = -w.cur_ver * (pnl + pl) - R(0.5) * vsg + pvt;
+__device__ __forceinline__ void vt_w(const CtxT<R> &c, const VtWeights<R> &w, int ji, int jk, int jl, ix_t i, R ps, R vsg, R pvt) {
+  R x = ps - R(0.5) * vsg + pvt;
   if (c.C.lmoist) {  // calc_p_grad_condensates_v, mo_p_grad.F90:106-120 (identically 0 when dry)
     const ix_t ia = LG_IX(c.G, ji, jk, jl - 1);
     const R da = c.w.pgc[ia];  // rho_gas/rho_sum - 1 of the old state, from k_temperature
@@ -747,7 +734,7 @@ __device__ __forceinline__ void vt_w(const CtxT<R> &c, const VtWeights<R> &w, in
     x = x + R(0.5) * (da + db) * c.g.gravity_m_v[i];
   }
   if (w.mom) x = x + c.w.mom_z[i];
-  c.w.tend_w[i] = w.old_w * c.w.tend_w[i] + w.new_w * x;
+  c.w.tend_w[i] = vt_mean<R>(w, c.w.tend_w, i, x);
 }
 template <class R>
 __device__ __forceinline__ void b_vec_tend(const CtxT<R> &c, const StateDev &old, const StateDev &nw, int rk, const Bid bid) {
@@ -756,9 +743,9 @@ __device__ __forceinline__ void b_vec_tend(const CtxT<R> &c, const StateDev &old
   if (jk > nx + 1 || ji > ny + 1 || jl > nl) return;
   const VtWeights<R> w = vt_weights(c, rk);
   const ix_t i = LG_IX(c.G, ji, jk, jl);
-  if (ji <= ny) vt_u(c, old, nw, w, i, c.w.pold_u[i], c.w.pnl_u[i], c.w.pl_u[i], c.w.vsg_x[i], c.w.pvt_x[i]);
-  if (jk <= nx) vt_v(c, old, nw, w, i, c.w.pold_v[i], c.w.pnl_v[i], c.w.pl_v[i], c.w.vsg_y[i], c.w.pvt_y[i]);
-  if (ji <= ny && jk <= nx && jl >= 2) vt_w(c, w, ji, jk, jl, i, c.w.pnl_w[i], c.w.pl_w[i], c.w.vsg_z[i], c.w.pvt_z[i]);
+  if (ji <= ny) vt_u(c, old, nw, w, i, c.w.ps_u[i], c.w.vsg_x[i], c.w.pvt_x[i]);
+  if (jk <= nx) vt_v(c, old, nw, w, i, c.w.ps_v[i], c.w.vsg_y[i], c.w.pvt_y[i]);
+  if (ji <= ny && jk <= nx && jl >= 2) vt_w(c, w, ji, jk, jl, i, c.w.ps_w[i], c.w.vsg_z[i], c.w.pvt_z[i]);
 }
 template <class R>
 __global__ void __launch_bounds__(BX * BY) k_vec_tend(const CtxT<R> c, const StateDev old, const StateDev nw, int rk) {
@@ -774,20 +761,20 @@ __device__ __forceinline__ void b_pgrad_vt(const CtxT<R> &c, const StateDev &old
   KIDX_ZFAST(c.G.nx, c.G.ny, c.G.nl);
   const int nx = c.G.nx, ny = c.G.ny;
   if (jk > nx || ji > ny || jl > c.G.nl) return;
-  const PGrad<R> g = pgrad_interior(c, old, lfirst, ji, jk, jl);
   const VtWeights<R> w = vt_weights(c, 1);
+  const PGrad<R> g = pgrad_interior(c, old, w, lfirst, ji, jk, jl);
   const ix_t i = LG_IX(c.G, ji, jk, jl);
-  vt_u(c, old, nw, w, i, g.old_u, g.nl_u, g.l_u, c.w.vsg_x[i], c.w.pvt_x[i]);
+  vt_u(c, old, nw, w, i, g.u, c.w.vsg_x[i], c.w.pvt_x[i]);
   if (jk == 1) {
     const ix_t iX = LG_IX(c.G, ji, nx + 1, jl);
-    vt_u(c, old, nw, w, iX, g.old_u, g.nl_u, g.l_u, c.w.vsg_x[iX], c.w.pvt_x[iX]);
+    vt_u(c, old, nw, w, iX, g.u, c.w.vsg_x[iX], c.w.pvt_x[iX]);
   }
-  vt_v(c, old, nw, w, i, g.old_v, g.nl_v, g.l_v, c.w.vsg_y[i], c.w.pvt_y[i]);
+  vt_v(c, old, nw, w, i, g.v, c.w.vsg_y[i], c.w.pvt_y[i]);
   if (ji == 1) {
     const ix_t iY = LG_IX(c.G, ny + 1, jk, jl);
-    vt_v(c, old, nw, w, iY, g.old_v, g.nl_v, g.l_v, c.w.vsg_y[iY], c.w.pvt_y[iY]);
+    vt_v(c, old, nw, w, iY, g.v, c.w.vsg_y[iY], c.w.pvt_y[iY]);
   }
-  if (jl >= 2) vt_w(c, w, ji, jk, jl, i, g.nl_w, g.l_w, c.w.vsg_z[i], c.w.pvt_z[i]);
+  if (jl >= 2) vt_w(c, w, ji, jk, jl, i, g.w, c.w.vsg_z[i], c.w.pvt_z[i]);
 }
 template <class R>
 __global__ void __launch_bounds__(BX * BY) k_pgrad_vt(const CtxT<R> c, const StateDev old, const StateDev nw, int lfirst) {
@@ -818,11 +805,11 @@ __device__ __forceinline__ void b_vort_flux_vt(const CtxT<R> &c, const StateDev 
     g.y_edge = ji == 1 ? c.w.vsg_y[iY] : R(0.0);
   }
   const VtWeights<R> w = vt_weights(c, 2);
-  vt_u(c, old, nw, w, i, c.w.pold_u[i], c.w.pnl_u[i], c.w.pl_u[i], g.x, f.x);
-  if (jk == 1) vt_u(c, old, nw, w, iX, c.w.pold_u[iX], c.w.pnl_u[iX], c.w.pl_u[iX], g.x_edge, f.x);
-  vt_v(c, old, nw, w, i, c.w.pold_v[i], c.w.pnl_v[i], c.w.pl_v[i], g.y, f.y);
-  if (ji == 1) vt_v(c, old, nw, w, iY, c.w.pold_v[iY], c.w.pnl_v[iY], c.w.pl_v[iY], g.y_edge, f.y);
-  if (jl >= 2) vt_w(c, w, ji, jk, jl, i, c.w.pnl_w[i], c.w.pl_w[i], g.z, f.z);
+  vt_u(c, old, nw, w, i, c.w.ps_u[i], g.x, f.x);
+  if (jk == 1) vt_u(c, old, nw, w, iX, c.w.ps_u[iX], g.x_edge, f.x);
+  vt_v(c, old, nw, w, i, c.w.ps_v[i], g.y, f.y);
+  if (ji == 1) vt_v(c, old, nw, w, iY, c.w.ps_v[iY], g.y_edge, f.y);
+  if (jl >= 2) vt_w(c, w, ji, jk, jl, i, c.w.ps_w[i], g.z, f.z);
 }
 template <class R>
 __global__ void __launch_bounds__(BX * BY) k_vort_flux_vt(const CtxT<R> c, const StateDev old, const StateDev nw, int with_ke_grad) {

@@ -118,3 +118,34 @@ def test_checkpoint_of_another_configuration_is_refused():
         a.restore(blob[:-8])
     a.close()
     b.close()
+
+
+def test_checkpoint_pressure_gradient_parts_are_summed():
+    """The layout has boxes for the nonlinear and the linear pressure gradient, whose sum is what a run
+    carries: a checkpoint that spreads the sum over both (halves, exact in binary) continues the
+    same run."""
+    cfg, g, st, _, _ = _restart_case("dry")
+    a = Step(cfg, g)
+    a.start(st)
+    a.run(0, 5)
+    slots = [a.get_state(0), a.get_state(1)]
+    blob = bytearray(a.checkpoint())
+    a.run(5, 4)
+    want = a.get_state(1)
+    a.close()
+    pitch = (cfg.nx + 1 + 15) // 16 * 16
+    box, head = 8 * (cfg.n_layers + 1) * (cfg.ny + 1) * pitch, 56
+    part = lambda q: np.frombuffer(blob, dtype=np.float64, count=box // 8, offset=head + q * box)  # noqa: E731
+    for nonlinear, linear in ((0, 3), (1, 4)):
+        assert np.abs(part(nonlinear)).max() > 0.0 and np.abs(part(linear)).max() == 0.0
+        half = 0.5 * part(nonlinear)
+        for q in (nonlinear, linear):
+            blob[head + q * box:head + (q + 1) * box] = half.tobytes()
+    b = Step(cfg, g)
+    b.set_state(0, slots[0])
+    b.set_state(1, slots[1])
+    b.restore(bytes(blob))
+    b.run(5, 4)
+    got = b.get_state(1)
+    b.close()
+    assert all(np.array_equal(got[f], want[f]) for f in want)
