@@ -17,12 +17,13 @@ namespace lgame {
 
 // PH_PGRAD is the first substep's pressure gradient with its wind update (b_pgrad_vt), PH_VORT_FLUX_VT
 // the second substep's vorticity flux term with its wind update (b_vort_flux_vt); PH_VEC_TEND is the
-// second substep's wind update alone (runs without momentum advection).
+// second substep's wind update alone (runs without momentum advection).  PH_VER_SEG takes the place of
+// PH_SOLVE_VER when ver_segments holds for every member.
 enum Phase : int {
   PH_TEMPERATURE, PH_SFC_TURB, PH_THETA_GRAD, PH_THETA_DIV, PH_THETA_EDGE, PH_PGRAD, PH_POT_VORT,
   PH_VORT_FLUX, PH_DIFF_ZETA, PH_DIFF_COEF, PH_DIFF_DUAL, PH_DIFF_MOM, PH_PBL_WIND,
   PH_DISSIPATION, PH_VEC_TEND, PH_DIFF_FLUX, PH_DIFF_DIV, PH_SCALAR, PH_SURFACE, PH_SOLVE_VER, PH_SOLVE_GEN, PH_RAD,
-  PH_VORT_FLUX_VT,
+  PH_VORT_FLUX_VT, PH_VER_SEG,
   PH_COUNT
 };
 
@@ -65,6 +66,7 @@ struct BatchArgs {
   int old_slot, new_slot;  // state_old and state_new
   int state_slot;          // the slot of the phase's state argument (state_old, or state_new at rk 2)
   int rk, lfirst, nfield, flags;
+  int nl_max;  // the most layers of a member
   int ke;  // the mass-flux kernel also forms the kinetic energy, the vorticity-flux kernel its gradient
 };
 
@@ -85,6 +87,7 @@ __host__ __device__ inline void phase_grid(int ph, const Geom &G, int by, int se
     case PH_DIFF_ZETA: ex = nx + 1; ey = ny + 1; flat = true; break;
     case PH_SCALAR: gx = ((nx + SCOL_CELLS - 1) / SCOL_CELLS) * ((ny + by - 1) / by) * seg; gy = gz = 1; return;
     case PH_SOLVE_VER: gx = col_waves(G); gy = gz = 1; return;
+    case PH_VER_SEG: gx = vs_blocks_per_row(G.nx) * G.ny; gy = gz = 1; return;
     case PH_RAD: gx = (nx * ny + BCOL - 1) / BCOL; gy = gz = 1; return;
     case PH_SOLVE_GEN: gx = (col_waves(G) + GEN_GROUPS - 1) / GEN_GROUPS; gy = gz = 1; return;
     default: return;

@@ -1459,8 +1459,9 @@ int lgame_autotune(lgame_handle *h, int steps, int *rows) {
     }
   }
   h->tiles.seg = best_seg;
-  // the vertical solver in one or three passes, on domains near the size where they trade places
-  if (!rc && h->c.G.nl >= 3 && col_waves(h->c.G) < 2 * VER_SPLIT_WAVES) {
+  // the vertical solver in one or three passes, on domains near the size where they trade places (the
+  // columns that k_ver_seg does not take)
+  if (!rc && !ver_segments(h->c.G.nl) && col_waves(h->c.G) < 2 * VER_SPLIT_WAVES) {
     int best_p = h->tiles.ver_passes;
     double best_p_ms = 1e300;
     for (int p : {1, 3}) {
@@ -1543,6 +1544,7 @@ struct BatchGroup {
   float *rx = nullptr, *ry = nullptr;  // the surrogate's inputs and outputs of every member's columns
   MlpWork *work = nullptr;
   long long cols = 0;
+  int nl_max = 0;                // layers of the tallest member
 };
 
 struct lgame_ensemble {
@@ -1576,7 +1578,7 @@ int efail(lgame_ensemble *e, int code, const char *fmt, ...) {
   } while (0)
 
 // A member's step as a branch of the ensemble's graph.  The branches run concurrently and fill the
-// GPU together, so the vertical solver takes its one-pass form (the three-pass form of a small
+// GPU together, so the vertical solver of tall columns takes its one-pass form (the three-pass form of a small
 // domain alone reads its inputs twice: the 48-member ensemble step took 74.2 instead of 71.8 ms).
 void enqueue_member(lgame_handle *h, int a, int b, int step, const RadCall *rad) {
   Tiles t = h->tiles;
@@ -1653,7 +1655,10 @@ int build_group(lgame_ensemble *e, BatchGroup &g) {
   ECHK(e, hipMalloc(&g.mem, g.mem_bytes));
   ECHK(e, hipMalloc(&g.prefix, sizeof(int) * PH_COUNT * (n + 1)));
   ECHK(e, hipEventCreateWithFlags(&g.uploaded, hipEventDisableTiming));
-  for (auto *h : g.m) g.cols += (long long)h->c.G.nx * h->c.G.ny;
+  for (auto *h : g.m) {
+    g.cols += (long long)h->c.G.nx * h->c.G.ny;
+    if (h->c.G.nl > g.nl_max) g.nl_max = h->c.G.nl;
+  }
   MemberDev<R> *M = static_cast<MemberDev<R> *>(g.host);
   // The column-marching scalar kernel cuts a small domain's columns into segments to fill the
   // GPU; in one launch over the whole group the members' rows fill it together, so the segments
@@ -1771,6 +1776,8 @@ int enqueue_group(lgame_ensemble *e, BatchGroup &g, int a_slot, int b_slot, int 
     dim3 blk(BX, 1, 1);
     if (ph == PH_SOLVE_VER)
       blk = dim3(BCOL);
+    else if (ph == PH_VER_SEG)
+      blk = dim3(VS_THREADS);
     else if (ph == PH_SOLVE_GEN)
       blk = dim3(BCOL, NTR * GEN_GROUPS);
     else
@@ -1782,7 +1789,7 @@ int enqueue_group(lgame_ensemble *e, BatchGroup &g, int a_slot, int b_slot, int 
     if (!batch_launch_step<R>(ph, grd, blk, st, M, pf, n, a) && !batch_launch_diff<R>(ph, grd, blk, st, M, pf, n, a))
       (void)batch_launch_solve<R>(ph, grd, blk, st, M, pf, n, a);
   };
-  BatchArgs base{a_slot, b_slot, a_slot, 1, step == 0 ? 1 : 0, 0, 0, C.llinear ? 0 : 1};
+  BatchArgs base{a_slot, b_slot, a_slot, 1, step == 0 ? 1 : 0, 0, 0, g.nl_max, C.llinear ? 0 : 1};
   launch(PH_TEMPERATURE, base);
   // update_sfc_turb_quantities and update_rad_fluxes with state_old (mo_manage_pchevi.F90:52-58)
   if (C.lsfc_turb) launch(PH_SFC_TURB, base);
@@ -1844,7 +1851,7 @@ int enqueue_group(lgame_ensemble *e, BatchGroup &g, int a_slot, int b_slot, int 
     }
     launch(PH_SCALAR, a);
     if (C.lsoil || C.lsens) launch(PH_SURFACE, a);
-    launch(PH_SOLVE_VER, a);
+    launch(ver_segments(g.nl_max) ? PH_VER_SEG : PH_SOLVE_VER, a);
     if (g.moist) launch(PH_SOLVE_GEN, a);
   }
   ECHK(e, hipGetLastError());

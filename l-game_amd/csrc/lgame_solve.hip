@@ -307,6 +307,211 @@ __global__ void __launch_bounds__(BCOL) k_solve_ver(const CtxT<R> c, const State
   b_solve_ver(c, old, nw, rk, bid_here());
 }
 
+// ---- the same solve with a column's levels cut into segments held in registers ------------------
+// A block owns VS_COLS columns of one row and cuts each into VS_SEG segments of consecutive layers,
+// one lane per (column, segment).  All lanes load their layers and form their rows of the system at
+// once; then only the Thomas recursion runs from segment to segment (the lanes of one segment at a
+// time, the eliminated coefficients of its last row through LDS), down and back up; then all lanes
+// form the new state.  Between the phases a lane keeps its rows, the explicit densities, gamma and
+// theta_v at the interfaces in registers and the old state and volume of its layers in LDS, so the
+// column scratch and the second reads of most inputs of ver_column are gone.  The expressions are
+// those of ver_column, so the results are the same bits.
+//
+// What bounds it: memory traffic and the divisions of the rows on large domains, the recursion's chain
+// of dependent divisions and the latency of one block on small ones.  A CU's registers and LDS hold 64
+// columns at 60 levels; as two blocks of 32 columns one runs its recursion while the other waits for
+// memory.  us per launch, mean of predictor and corrector, ver_column (three passes for the dry
+// ones) -> here: 512x512x60 FP64 841 -> 577, mixed 776 -> 560; dry 161x129x47 FP64 93 -> 66, dry
+// 128x128x50 mixed 64 -> 38; dry 201x3x40 FP64 20.1 -> 18.5.
+// Keeps the compiler from moving the computation of these values below this point (it would sink a row
+// of the system to its first use and keep all of the row's inputs in registers until then).
+__device__ __forceinline__ void pin(double &a, double &b, double &c, double &d) {
+  asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+}
+
+// K: most layers of a segment
+template <class R, int RK, int K>
+__device__ __forceinline__ void ver_segment(const CtxT<R> &c, const StateDev &old, const StateDev &nw, int ji, int jk_raw, double *lds) {
+  const int nl = c.G.nl, g = c.G.ncond;
+  const StateDev &nu = RK == 1 ? old : nw;
+  const double dt = c.C.dtime;
+  const int col = (int)threadIdx.x % VS_COLS, seg = (int)threadIdx.x / VS_COLS;
+  const bool active = jk_raw <= c.G.nx;
+  const int jk = active ? jk_raw : c.G.nx;  // idle lanes mirror the last column and store nothing
+  // this lane's layers l0..l0+len-1 and rows l0..l0+nrow-1 (row q couples layers q and q+1)
+  const int l0 = 1 + nl * seg / VS_SEG, len = nl * (seg + 1) / VS_SEG + 1 - l0;
+  const int nrow = l0 + len - 1 == nl ? len - 1 : len;
+  double *const s_rho = lds, *const s_rt = s_rho + VS_COLS * nl, *const s_rhoe = s_rt + VS_COLS * nl, *const s_rte = s_rhoe + VS_COLS * nl;
+  double *const xch = s_rte + VS_COLS * nl;
+  auto sl = [&](int l) { return (l - 1) * VS_COLS + col; };  // a layer's place in the LDS arrays
+  const ix_t i0 = LG_IX(c.G, ji, jk, 1), lvl = (ix_t)c.G.lvl;
+  auto ix = [&](int l) { return i0 + (ix_t)((l < nl ? l : nl) - 1) * lvl; };  // (past the bottom: layer nl, not used)
+
+  double d[K], r[K], cc[K], e[K], tin[K], ga[K];
+  {
+    Layer L0 = make_layer(load_raw(c, old, nu, RK, ix(l0)), RK, dt);
+    const RawLayer raw1 = load_raw(c, old, nu, RK, ix(l0 + 1));
+    Layer L1 = make_layer(raw1, RK, dt);
+    Iface F0 = make_iface(L0, L1, raw1);
+    // the next layer's inputs are in flight while a row is formed, where the registers allow it
+    // (K = 8: 580 -> 544 us at 512x512x60 FP64; with K = 9 they would spill)
+    constexpr bool ahead = K <= 8;
+    RawLayer nxt;
+    if (ahead) nxt = load_raw(c, old, nu, RK, ix(l0 + 2));
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (ahead && k * VS_SEG >= nl) break;  // longer than this column's segments
+      RawLayer cur;  // layer l0+k+2
+      if (ahead) {
+        cur = nxt;
+        if (k + 1 < K) nxt = load_raw(c, old, nu, RK, ix(l0 + k + 3));
+      } else {
+        cur = load_raw(c, old, nu, RK, ix(l0 + k + 2));
+      }
+      const Layer L2 = make_layer(cur, RK, dt);
+      const Iface F1 = make_iface(L1, L2, cur);
+      const Row w = make_row(L0, L1, L2, F0, F1, l0 + k + 2 <= nl, dt);
+      d[k] = w.d;
+      r[k] = w.r;
+      cc[k] = w.c;
+      e[k] = w.e;
+      tin[k] = F0.tin;
+      ga[k] = L0.ga;
+      pin(d[k], r[k], cc[k], e[k]);
+      if (k < len) {
+        s_rho[sl(l0 + k)] = L0.rho_o;
+        s_rt[sl(l0 + k)] = L0.rt_o;
+        s_rhoe[sl(l0 + k)] = L0.rhoe;
+        s_rte[sl(l0 + k)] = L0.rte;
+      }
+      L0 = L1;
+      L1 = L2;
+      F0 = F1;
+      __builtin_amdgcn_sched_barrier(0);  // one layer's loads in flight: hoisting more of them spills
+    }
+  }
+  // thomas_algorithm, mo_column_solvers.F90:622-632 (with ep = c = rp = 0 before row 1, whose first
+  // row is then e/d and r/d)
+  double *const x_ep = xch, *const x_rp = xch + VS_COLS, *const x_c = xch + 2 * VS_COLS;
+  for (int s = 0; s < VS_SEG; ++s) {
+    if (seg == s && nrow > 0) {
+      double ep = 0.0, rp = 0.0, cp = 0.0;
+      if (s > 0 && l0 > 1) {
+        ep = x_ep[col];
+        rp = x_rp[col];
+        cp = x_c[col];
+      }
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+        if (k < nrow) {
+          const double den = d[k] - ep * cp;
+          ep = e[k] / den;
+          rp = (r[k] - rp * cp) / den;
+          cp = cc[k];
+          e[k] = ep;
+          r[k] = rp;
+        }
+      x_ep[col] = ep;
+      x_rp[col] = rp;
+      x_c[col] = cp;
+    }
+    __syncthreads();
+  }
+  // the inputs of the new state that were not kept, in flight during the back substitution
+  double tb[K], az[K], wo[K], Vl[K], epo[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    tb[k] = c.g64.theta_v_bg[ix(l0 + k)];
+    Vl[k] = c.g64.volume[ix(l0 + k)];
+    epo[k] = old.exner_pert[ix(l0 + k)];
+    const ix_t ib = ix(l0 + k + 1);
+    az[k] = c.g64.area_z[ib];
+    wo[k] = old.wind_w[ib];
+  }
+  // back substitution (mo_column_solvers.F90:635-638, after the last barrier of the elimination): r becomes x.  Per segment, the solution and
+  // theta_v at its last row go to the next segment, whose first layer lies below it.
+  double *const x_x = xch, *const x_tin = xch + VS_COLS * VS_SEG, *const x_rho = xch + 2 * VS_COLS * VS_SEG;
+  double *const x_low_s = xch + 3 * VS_COLS * VS_SEG;
+  for (int s = VS_SEG - 1; s >= 0; --s) {
+    if (seg == s && nrow > 0) {
+      double x = l0 + nrow - 1 == nl - 1 ? 0.0 : x_low_s[col];
+      double x_last = 0.0, t_last = 0.0;
+#pragma unroll
+      for (int k = K - 1; k >= 0; --k)
+        if (k < nrow) {
+          x = l0 + k == nl - 1 ? r[k] : r[k] - e[k] * x;
+          r[k] = x;
+          if (k == nrow - 1) {
+            x_last = x;
+            t_last = tin[k];
+          }
+        }
+      x_low_s[col] = x;
+      x_x[s * VS_COLS + col] = x_last;
+      x_tin[s * VS_COLS + col] = t_last;
+    }
+    __syncthreads();
+  }
+  // the new state (mo_column_solvers.F90:305-349); cc becomes the new density
+  double x_above = 0.0, t_above = 0.0;
+  if (l0 > 1 && len > 0) {  // the row above the segment, of the nearest segment above that has rows
+    int s = seg - 1;
+    while (nl * s / VS_SEG == nl * (s + 1) / VS_SEG) --s;
+    x_above = x_x[s * VS_COLS + col];
+    t_above = x_tin[s * VS_COLS + col];
+  }
+  bool finite = true;
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    if (k < len) {
+      const int Lr = l0 + k;
+      const double V = Vl[k], rt_o = s_rt[sl(Lr)];
+      const double x_up = k > 0 ? r[k > 0 ? k - 1 : 0] : x_above, tin_u = k > 0 ? tin[k > 0 ? k - 1 : 0] : t_above;
+      double rho_new, rt_new;
+      new_densities(Lr, nl, s_rhoe[sl(Lr)], s_rte[sl(Lr)], V, dt, x_up, r[k], tin_u, tin[k], rho_new, rt_new);
+      const double ep_new = epo[k] + V * ga[k] * (rt_new - rt_o);
+      const double tp_new = rt_new / rho_new - tb[k];
+      cc[k] = rho_new;
+      if (active) {
+        const ix_t i = ix(Lr);
+        nw.rho[g][i] = rho_new;
+        nw.rhotheta_v[i] = rt_new;
+        nw.exner_pert[i] = ep_new;
+        nw.theta_v_pert[i] = tp_new;
+      }
+      if (RK == 2) finite = finite && isfinite(rho_new) && isfinite(rt_new) && isfinite(ep_new) && isfinite(tp_new);
+    }
+  if (len > 0) x_rho[seg * VS_COLS + col] = cc[0];
+  __syncthreads();
+  // w at the interface below each layer, level Lr+1
+  double rho_next = 0.0;  // new rho of the first layer below the segment
+  if (l0 + len - 1 < nl && len > 0) {
+    int s = seg + 1;
+    while (nl * s / VS_SEG == nl * (s + 1) / VS_SEG) ++s;
+    rho_next = x_rho[s * VS_COLS + col];
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    if (k < nrow) {
+      const double rho_b = k + 1 < len ? cc[k + 1 < K ? k + 1 : k] : rho_next;
+      const double rio = 0.5 * (s_rho[sl(l0 + k)] + s_rho[sl(l0 + k + 1)]);
+      const double rin = 0.5 * (cc[k] + rho_b);
+      if (active) nw.wind_w[ix(l0 + k + 1)] = (2.0 * r[k] / az[k] - rin * wo[k]) / rio;
+    }
+  if (RK == 2 && !finite && active) atomicOr(c.C.nonfinite, 1ull);
+}
+template <class R, int RK, int K>
+__device__ __forceinline__ void b_ver_seg(const CtxT<R> &c, const StateDev &old, const StateDev &nw, const Bid bid, double *lds) {
+  const int bpr = vs_blocks_per_row(c.G.nx);
+  const int ji = bid.x / bpr + 1, jk = (bid.x % bpr) * VS_COLS + (int)threadIdx.x % VS_COLS + 1;
+  ver_segment<R, RK, K>(c, old, nw, ji, jk, lds);
+}
+template <class R, int RK, int K>
+__global__ void __launch_bounds__(VS_THREADS, 2) k_ver_seg(const CtxT<R> c, const StateDev old, const StateDev nw) {
+  extern __shared__ double lds[];
+  b_ver_seg<R, RK, K>(c, old, nw, bid_here(), lds);
+}
+
 // ---- the same solve in three passes, for domains with fewer column wavefronts than SIMDs -------
 // On such a domain k_solve_ver's wavefronts leave SIMDs idle and each runs its column's chain of
 // dependent FP64 operations alone.  Here the rows of the system (k_ver_rows) and the new state
@@ -483,9 +688,29 @@ __global__ void __launch_bounds__(BX * 4) k_ver_update(const CtxT<R> c, const St
     atomicOr(c.C.nonfinite, 1ull);
 }
 
+// the instantiation for columns of up to nl layers
+#define LG_VS_DISPATCH(nl)                 \
+  do {                                     \
+    if ((nl) <= 5 * VS_SEG) LG_VS(5);      \
+    else if ((nl) <= 8 * VS_SEG) LG_VS(8); \
+    else LG_VS(9);                         \
+  } while (0)
+
 template <class R>
 void launch_solve_ver(const CtxT<R> &c, const StateDev &old, const StateDev &nw, int rk, int passes, hipStream_t st) {
   const Geom &G = c.G;
+  if (ver_segments(G.nl)) {
+    const dim3 g((unsigned)(vs_blocks_per_row(G.nx) * G.ny)), b(VS_THREADS);
+    const size_t l = vs_lds_bytes(G.nl);
+#define LG_VS(K)                                                                                   \
+  do {                                                                                             \
+    if (rk == 1) hipLaunchKernelGGL((k_ver_seg<R, 1, K>), g, b, l, st, c, old, nw);                \
+    else hipLaunchKernelGGL((k_ver_seg<R, 2, K>), g, b, l, st, c, old, nw);                        \
+  } while (0)
+    LG_VS_DISPATCH(G.nl);
+#undef LG_VS
+    return;
+  }
   if (passes != 3 || G.nl < 3) {
     hipLaunchKernelGGL(k_solve_ver<R>, dim3((unsigned)col_waves(G)), dim3(BCOL), 0, st, c, old, nw, rk);
     return;
@@ -881,12 +1106,30 @@ template __global__ void k_solve_gen<float>(const CtxT<float>, const StateDev, c
 
 // ---- the same kernels over a group of domains (one launch per phase) ------------------------
 LG_BATCH_KERNEL(solve_ver, BCOL, PH_SOLVE_VER, b_solve_ver(d.c, d.s[a.old_slot], d.s[a.new_slot], a.rk, bid))
+template <class R, int RK, int K>
+__global__ void __launch_bounds__(VS_THREADS, 2)
+    kb_ver_seg(const MemberDev<R> *__restrict__ M, const int *__restrict__ prefix, int nm, const BatchArgs a) {
+  extern __shared__ double lds[];
+  Bid bid;
+  const MemberDev<R> &d = batch_block(M, prefix, nm, PH_VER_SEG, bid);
+  b_ver_seg<R, RK, K>(d.c, d.s[a.old_slot], d.s[a.new_slot], bid, lds);
+}
 LG_BATCH_KERNEL(solve_gen, BCOL * NTR * GEN_GROUPS, PH_SOLVE_GEN, b_solve_gen(d.c, d.s[a.old_slot], d.s[a.new_slot], a.rk, bid))
 
 template <class R>
 bool batch_launch_solve(int ph, dim3 g, dim3 b, hipStream_t st, const MemberDev<R> *M, const int *prefix, int nm, const BatchArgs &a) {
   if (ph == PH_SOLVE_VER) {
     hipLaunchKernelGGL(kb_solve_ver<R>, g, b, 0, st, M, prefix, nm, a);
+    return true;
+  }
+  if (ph == PH_VER_SEG) {  // a.nl_max: the layers of the group's tallest column
+#define LG_VS(K)                                                                                                 \
+  do {                                                                                                           \
+    if (a.rk == 1) hipLaunchKernelGGL((kb_ver_seg<R, 1, K>), g, b, vs_lds_bytes(a.nl_max), st, M, prefix, nm, a); \
+    else hipLaunchKernelGGL((kb_ver_seg<R, 2, K>), g, b, vs_lds_bytes(a.nl_max), st, M, prefix, nm, a);           \
+  } while (0)
+    LG_VS_DISPATCH(a.nl_max);
+#undef LG_VS
     return true;
   }
   if (ph == PH_SOLVE_GEN) {

@@ -77,8 +77,22 @@ template <class R>
 void launch_scalar_col(const CtxT<R> &c, const StateDev &ss, const StateDev &nw, int rk, int rows, int nseg, hipStream_t st);
 // Lanes per block of the column solvers.
 constexpr int BCOL = 64;
-// The vertical solver runs in three passes (rows, Thomas recursion per column, new state) on
-// domains with fewer column wavefronts than this, the 1024 SIMDs of the MI355X.
+// The vertical solver with a column's levels cut into segments held in registers (k_ver_seg): columns
+// per block, segments per column.
+constexpr int VS_COLS = 32, VS_SEG = 8;
+constexpr int VS_THREADS = VS_COLS * VS_SEG;
+constexpr int VS_LDS = 4;   // arrays of a column kept in LDS: old rho, rhotheta_v, Exner pressure and the volume
+constexpr int VS_XCH = 3 * VS_SEG + 1;  // doubles per column exchanged between segments
+// bytes of LDS a block needs for nl levels
+__host__ __device__ inline size_t vs_lds_bytes(int nl) { return sizeof(double) * VS_COLS * ((size_t)VS_LDS * nl + VS_XCH); }
+__host__ __device__ inline int vs_blocks_per_row(int nx) { return (nx + VS_COLS - 1) / VS_COLS; }
+// Columns of at most VS_MAX_NL layers take this kernel, whatever the domain's size (it was faster from
+// 12 to 4096 column wavefronts); beyond, the segments' registers and LDS no longer let two blocks share
+// a CU and the column kernels below run.
+constexpr int VS_MAX_NL = 9 * VS_SEG;
+inline bool ver_segments(int nl) { return nl <= VS_MAX_NL; }
+// Taller columns: three passes (rows, Thomas recursion per column, new state) on domains with fewer
+// column wavefronts than this, the 1024 SIMDs of the MI355X, else one pass per column.
 constexpr int VER_SPLIT_WAVES = 1024;
 template <class R>
 void launch_solve_ver(const CtxT<R> &c, const StateDev &old, const StateDev &nw, int rk, int passes, hipStream_t st);

@@ -97,6 +97,43 @@ def test_vertical_solver_passes_keep_results(name):
     s.close()
 
 
+@pytest.mark.parametrize("nl,nx,moist", [(3, 4, False), (7, 31, False), (8, 32, True), (9, 33, False), (40, 65, False), (41, 5, True),
+                                         (64, 34, False), (65, 7, False), (72, 33, True), (73, 33, False)])
+def test_vertical_solver_segments_match_oracle(nl, nx, moist):
+    """The vertical solver cuts columns of up to 72 layers into 8 segments (empty ones below 8 layers)
+    in blocks of 32 columns: the edges of its layer ranges and of its blocks, bitwise against the
+    oracle."""
+    cfg = tiny_config(ny=4, nx=nx, n_layers=nl, moist=moist, freeslip=nl % 2 == 1)
+    g, st = make_case(cfg, cloud_frac=0.2 if moist else 0.0)
+    want = _oracle(cfg, g, st, 3)
+    s = Step(cfg, g)
+    s.start(st)
+    s.run(0, 3)
+    got = s.get_state(1)
+    s.close()
+    assert all(np.array_equal(got[k], want[k]) for k in want)
+
+
+@pytest.mark.parametrize("layers", [(6, 44, 70), (6, 20, 73)])
+def test_batched_vertical_solver_with_members_of_different_height(layers):
+    cfgs = [tiny_config(ny=4 + i, nx=30 + 3 * i, n_layers=nl) for i, nl in enumerate(layers)]
+    cases = [make_case(c) for c in cfgs]
+    steps = []
+    for c, (g, st) in zip(cfgs, cases):
+        s = Step(c, g)
+        s.start(st)
+        steps.append(s)
+    e = Ensemble(steps)
+    e.run(0, 3, mode=Ensemble.BATCHED)
+    e.sync()
+    for c, (g, st), s in zip(cfgs, cases, steps):
+        got, want = s.get_state(1), _oracle(c, g, st, 3)
+        assert all(np.array_equal(got[k], want[k]) for k in want), c.n_layers
+    e.close()
+    for s in steps:
+        s.close()
+
+
 def test_vertical_solver_default_passes_by_size():
     """One pass per column once the domain has as many 64-column wavefronts as the GPU has SIMDs."""
     for n, want in ((128, 3), (256, 1)):
