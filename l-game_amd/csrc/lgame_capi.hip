@@ -371,7 +371,7 @@ int enqueue_pchevi(const CtxT<R> &c, const StateDev &old, const StateDev &nw, in
       LG_LAUNCH_ZFAST(KI_DIFF_MOM, k_diff_mom, nx, ny, nl, c, old);
     }
     if (rk == 1 && c.C.lpbl) LG_LAUNCH(KI_DIFF_DUAL, k_pbl_wind, nx, ny, 1, c, old);
-    if (rk == 1 && diss_levels(c) > 0) LG_LAUNCH(KI_DISSIPATION, k_dissipation, nx, ny, diss_levels(c), c, old);
+    if (rk == 1 && !klemp_only(c) && diss_levels(c) > 0) LG_LAUNCH(KI_DISSIPATION, k_dissipation, nx, ny, diss_levels(c), c, old);
     // the first substep's pressure gradient (manage_p_grad) and, from its values, the wind update;
     // no kernel in between reads or writes what the pressure gradient uses or forms
     if (rk == 1)
@@ -1834,7 +1834,7 @@ int enqueue_group(lgame_ensemble *e, BatchGroup &g, int a_slot, int b_slot, int 
     if (rk == 1 && C.lmom_h)
       for (int ph : {PH_DIFF_ZETA, PH_DIFF_COEF, PH_DIFF_DUAL, PH_DIFF_MOM}) launch(ph, a);
     if (rk == 1 && C.lpbl) launch(PH_PBL_WIND, a);
-    if (rk == 1 && (C.lklemp || C.lmom_h || C.lmom_v || C.lpbl)) launch(PH_DISSIPATION, a);
+    if (rk == 1 && (C.lmom_h || C.lmom_v || C.lpbl)) launch(PH_DISSIPATION, a);  // (the Klemp layer alone: PH_TEMPERATURE)
     if (rk == 1)
       launch(PH_PGRAD, a);  // the pressure gradient with the wind update
     else if (!winds_done)

@@ -109,13 +109,19 @@ constexpr int GEN_GROUPS = 2;  // 64-column groups per block
 
 // Levels 1..diss_levels in which k_dissipation forms the dissipation rate: with a friction of the wind
 // all of them, with the Klemp layer alone those whose upper or lower interface lies in it (below it
-// every term has a zero factor, the array keeps its initial zeros and is not read), else none.  At
-// 512x512x60 with 24 levels in the layer the FP64 launch takes 115 instead of 249 us.
+// every term has a zero factor, the array keeps its initial zeros and is not read), else none.
 template <class R>
 __host__ __device__ inline int diss_levels(const CtxT<R> &c) {
   if (c.C.lmom_h || c.C.lmom_v || c.C.lpbl) return c.G.nl;
   if (!c.C.lklemp) return 0;
   return c.C.n_damping_levels < c.G.nl ? c.C.n_damping_levels : c.G.nl;
+}
+// The Klemp layer is the only dissipation: k_temperature, which holds the cell's density sum, forms the
+// rate as well, and k_dissipation is not launched (its launch over the 24 levels of the layer at
+// 512x512x60 took 115 us in FP64 and 102 in the mixed form; in k_temperature the rate adds 30 and 32).
+template <class R>
+__host__ __device__ inline bool klemp_only(const CtxT<R> &c) {
+  return c.C.lklemp && !c.C.lmom_h && !c.C.lmom_v && !c.C.lpbl;
 }
 
 // Optional timing hook around kernel groups (0 = vertical solver, 1 = tracer solver, 2 = step,

@@ -11,6 +11,37 @@
 
 namespace lgame {
 
+// the heating rate of simple_dissipation_rate (mo_momentum_diff_diss.F90:333-377) in one cell: minus the
+// density times the inner product of the wind with the momentum diffusion tendencies, whose vertical
+// parts at the cell's two levels are mz0, mz1 plus the Klemp layer's acceleration
+template <class R>
+__device__ __forceinline__ R klemp_heating(const CtxT<R> &c, const StateDev &s, int ji, int jk, int jl, R mz0, R mz1, R rs) {
+  const Geom &G = c.G;
+  const ix_t i = LG_IX(G, ji, jk, jl), ib = LG_IX(G, ji, jk, jl + 1);
+  R wk0 = mz0, wk1 = mz1;
+  const R dt = R(c.C.dtime);
+  if (c.C.lklemp && jl >= 2 && jl <= c.C.n_damping_levels) {
+    const R w = R(s.wind_w[i]);
+    const R k = (w / c.g.klemp_pref[i] - w) / dt;
+    wk0 = c.C.lmom_v ? wk0 + k : k;
+  }
+  if (c.C.lklemp && jl + 1 <= c.C.n_damping_levels) {
+    const R w = R(s.wind_w[ib]);
+    const R k = (w / c.g.klemp_pref[ib] - w) / dt;
+    wk1 = c.C.lmom_v ? wk1 + k : k;
+  }
+  R ip;
+  if (c.C.lmom_h || c.C.lpbl) {
+    ip = AT(c.g.ipw[0], ji, jk, jl) * ATR(s.wind_u, ji, jk + 1, jl) * AT(c.w.mom_x, ji, jk + 1, jl) +
+         c.g.ipw[1][i] * R(s.wind_v[i]) * c.w.mom_y[i] + c.g.ipw[2][i] * R(s.wind_u[i]) * c.w.mom_x[i] +
+         AT(c.g.ipw[3], ji, jk, jl) * ATR(s.wind_v, ji + 1, jk, jl) * AT(c.w.mom_y, ji + 1, jk, jl) +
+         c.g.ipw[4][i] * R(s.wind_w[i]) * wk0 + c.g.ipw[5][i] * R(s.wind_w[ib]) * wk1;
+  } else {  // the horizontal terms are products with zero tendencies
+    ip = c.g.ipw[4][i] * R(s.wind_w[i]) * wk0 + c.g.ipw[5][i] * R(s.wind_w[ib]) * wk1;
+  }
+  return -rs * ip;
+}
+
 // ---------------------------------------------------------------------------------------------
 // temperature_diagnostics, mo_derived.F90:18-38
 // ---------------------------------------------------------------------------------------------
@@ -35,6 +66,9 @@ __device__ __forceinline__ void b_temperature(const CtxT<R> &c, const StateDev &
     c.w.pgc[i] = rg / rs - R(1.0);
     c.w.vfall_cw[i] = v_fall_liquid(c, s, ji, jk, jl, (double)t, CLOUD_WATER_RADIUS);
   }
+  // simple_dissipation_rate with the Klemp layer alone: a product of this cell's values (with a
+  // friction of the wind it follows the momentum diffusion, k_dissipation)
+  if (klemp_only(c) && jl <= diss_levels(c)) c.w.heating_diss[i] = klemp_heating(c, s, ji, jk, jl, R(0.0), R(0.0), rs);
 }
 template <class R>
 __global__ void __launch_bounds__(BX * BY) k_temperature(const CtxT<R> c, const StateDev s) {
@@ -665,29 +699,8 @@ __device__ __forceinline__ void b_dissipation(const CtxT<R> &c, const StateDev &
     if (jl < nl) mz1 = (sp_c - sp(jl + 1)) / c.g.dz[ib] / (R(0.5) * (c.w.rsum[i] + c.w.rsum[ib]));
   }
   if (!c.C.lklemp && !c.C.lmom_h && !c.C.lpbl) return;  // mo_vector_tend_expl.F90:123-125
-  R wk0 = mz0, wk1 = mz1;
-  const R dt = R(c.C.dtime);
-  if (c.C.lklemp && jl >= 2 && jl <= c.C.n_damping_levels) {
-    const R w = R(s.wind_w[i]);
-    const R k = (w / c.g.klemp_pref[i] - w) / dt;
-    wk0 = c.C.lmom_v ? wk0 + k : k;
-  }
-  if (c.C.lklemp && jl + 1 <= c.C.n_damping_levels) {
-    const R w = R(s.wind_w[ib]);
-    const R k = (w / c.g.klemp_pref[ib] - w) / dt;
-    wk1 = c.C.lmom_v ? wk1 + k : k;
-  }
-  R ip;
-  if (c.C.lmom_h || c.C.lpbl) {
-    ip = AT(c.g.ipw[0], ji, jk, jl) * ATR(s.wind_u, ji, jk + 1, jl) * AT(c.w.mom_x, ji, jk + 1, jl) +
-         c.g.ipw[1][i] * R(s.wind_v[i]) * c.w.mom_y[i] + c.g.ipw[2][i] * R(s.wind_u[i]) * c.w.mom_x[i] +
-         AT(c.g.ipw[3], ji, jk, jl) * ATR(s.wind_v, ji + 1, jk, jl) * AT(c.w.mom_y, ji + 1, jk, jl) +
-         c.g.ipw[4][i] * R(s.wind_w[i]) * wk0 + c.g.ipw[5][i] * R(s.wind_w[ib]) * wk1;
-  } else {  // the horizontal terms are products with zero tendencies
-    ip = c.g.ipw[4][i] * R(s.wind_w[i]) * wk0 + c.g.ipw[5][i] * R(s.wind_w[ib]) * wk1;
-  }
   const R rs = (c.C.lmom_h || c.C.lmom_v) ? c.w.rsum[i] : rho_sum(c, s, i);
-  c.w.heating_diss[i] = -rs * ip;
+  c.w.heating_diss[i] = klemp_heating(c, s, ji, jk, jl, mz0, mz1, rs);
 }
 template <class R>
 __global__ void __launch_bounds__(BX * BY) k_dissipation(const CtxT<R> c, const StateDev s) {
@@ -711,7 +724,7 @@ __device__ __forceinline__ void vt_u(const CtxT<R> &c, const StateDev &old, cons
   R x = ps - R(0.5) * vsg + pvt;
   if (w.mom) x = x + c.w.mom_x[i];
   const R t = vt_mean<R>(w, c.w.tend_u, i, x);
-  c.w.tend_u[i] = t;
+  if (w.first) c.w.tend_u[i] = t;  // read by the second substep only
   nw.wind_u[i] = old.wind_u[i] + c.C.dtime * (double)t;  // FP64 state update
 }
 template <class R>
@@ -720,7 +733,7 @@ __device__ __forceinline__ void vt_v(const CtxT<R> &c, const StateDev &old, cons
   R x = ps - R(0.5) * vsg + pvt;
   if (w.mom) x = x + c.w.mom_y[i];
   const R t = vt_mean<R>(w, c.w.tend_v, i, x);
-  c.w.tend_v[i] = t;
+  if (w.first) c.w.tend_v[i] = t;
   nw.wind_v[i] = old.wind_v[i] + c.C.dtime * (double)t;
 }
 // the w point of cell (ji, jk, jl), jl >= 2
