@@ -22,7 +22,7 @@ namespace lgame {
 enum Phase : int {
   PH_TEMPERATURE, PH_SFC_TURB, PH_THETA_GRAD, PH_THETA_DIV, PH_THETA_EDGE, PH_PGRAD, PH_POT_VORT,
   PH_VORT_FLUX, PH_DIFF_ZETA, PH_DIFF_COEF, PH_DIFF_DUAL, PH_DIFF_MOM, PH_PBL_WIND,
-  PH_DISSIPATION, PH_VEC_TEND, PH_DIFF_FLUX, PH_DIFF_DIV, PH_SCALAR, PH_SURFACE, PH_SOLVE_VER, PH_SOLVE_GEN, PH_RAD,
+  PH_DISSIPATION, PH_VEC_TEND, PH_DIFF_FLUX, PH_SCALAR, PH_SURFACE, PH_SOLVE_VER, PH_SOLVE_GEN, PH_RAD,
   PH_VORT_FLUX_VT, PH_VER_SEG,
   PH_COUNT
 };
@@ -44,7 +44,6 @@ inline int phase_tile(int ph) {
     case PH_DISSIPATION: return KI_DISSIPATION;
     case PH_VEC_TEND: return KI_VEC_TEND;
     case PH_DIFF_FLUX: return KI_DIFF_FLUX;
-    case PH_DIFF_DIV: return KI_DIFF_DIV;
     case PH_SCALAR: return KI_SCALAR_DIV;
     default: return -1;
   }
@@ -82,10 +81,10 @@ __host__ __device__ inline void phase_grid(int ph, const Geom &G, int by, int se
     case PH_TEMPERATURE: case PH_THETA_DIV: case PH_DIFF_DUAL: case PH_DISSIPATION: break;
     case PH_SFC_TURB: case PH_PBL_WIND: case PH_SURFACE: ez = 1; break;
     case PH_THETA_GRAD: case PH_THETA_EDGE: case PH_VEC_TEND: ex = nx + 1; ey = ny + 1; break;
-    case PH_PGRAD: case PH_VORT_FLUX: case PH_VORT_FLUX_VT: case PH_DIFF_COEF: case PH_DIFF_MOM: case PH_DIFF_FLUX: case PH_DIFF_DIV: flat = true; break;
+    case PH_PGRAD: case PH_VORT_FLUX: case PH_VORT_FLUX_VT: case PH_DIFF_COEF: case PH_DIFF_MOM: flat = true; break;
     case PH_POT_VORT: ez = nlev; flat = true; break;
     case PH_DIFF_ZETA: ex = nx + 1; ey = ny + 1; flat = true; break;
-    case PH_SCALAR: gx = ((nx + SCOL_CELLS - 1) / SCOL_CELLS) * ((ny + by - 1) / by) * seg; gy = gz = 1; return;
+    case PH_SCALAR: case PH_DIFF_FLUX: gx = ((nx + SCOL_CELLS - 1) / SCOL_CELLS) * ((ny + by - 1) / by) * seg; gy = gz = 1; return;
     case PH_SOLVE_VER: gx = col_waves(G); gy = gz = 1; return;
     case PH_VER_SEG: gx = vs_blocks_per_row(G.nx) * G.ny; gy = gz = 1; return;
     case PH_RAD: gx = (nx * ny + BCOL - 1) / BCOL; gy = gz = 1; return;
@@ -152,6 +151,11 @@ LG_BATCH_LAUNCHER(batch_launch_solve)
 template <class R>
 void batch_launch_scalar(dim3 g, dim3 b, hipStream_t st, const MemberDev<R> *M, const int *prefix, int nm, const BatchArgs &a,
                          bool tr, bool o3, bool diff);
+
+// the diffusion column kernel, with its moist, temperature and density variants chosen by tr, temp, mass
+template <class R>
+void batch_launch_diff_col(dim3 g, dim3 b, hipStream_t st, const MemberDev<R> *M, const int *prefix, int nm, const BatchArgs &a,
+                           bool tr, bool temp, bool mass);
 
 // the radiation phases (all on the PH_RAD grid)
 enum RadPhase : int { RPH_SOLVER, RPH_GATHER, RPH_APPLY, RPH_SELECT };

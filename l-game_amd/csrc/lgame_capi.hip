@@ -382,18 +382,9 @@ int enqueue_pchevi(const CtxT<R> &c, const StateDev &old, const StateDev &nw, in
     // 60-99).  The temperature diffusion of the second substep repeats the first one with the same
     // temperature and coefficients, so its result is kept.
     if (rk == 1 && (c.C.ltemp_h || c.C.lmass_h)) {
-      if (nx % 2 == 0)
-        LG_LAUNCH_ZFAST(KI_DIFF_FLUX, k_diff_flux2, nx / 2, ny, nl, c, old);
-      else
-        LG_LAUNCH_ZFAST(KI_DIFF_FLUX, k_diff_flux, nx, ny, nl, c, old);
-      if constexpr (sizeof(R) == 8) {
-        if (nx % 2 == 0)
-          LG_LAUNCH_ZFAST(KI_DIFF_DIV, k_diff_div2, nx / 2, ny, nl, c);
-        else
-          LG_LAUNCH_ZFAST(KI_DIFF_DIV, k_diff_div, nx, ny, nl, c);
-      } else {
-        LG_LAUNCH_ZFAST(KI_DIFF_DIV, k_diff_div, nx, ny, nl, c);
-      }
+      if (pk) prof->begin(PROF_KERNEL0 + KI_DIFF_FLUX);
+      launch_diff_col(c, old, tiles.by[KI_DIFF_FLUX], tiles.seg, st);
+      if (pk) prof->end(PROF_KERNEL0 + KI_DIFF_FLUX);
     }
     // scalar_tend_expl (mo_scalar_tend_expl.F90:24-181); at rk 1 the theta_v edge values of the
     // pressure gradient are reused (same state, same winds)
@@ -716,7 +707,7 @@ int lgame_init(const lgame_dims *dims, const lgame_cfg *cfg, const lgame_grid_vi
   constexpr int NGRID = 40;
   const size_t fs = (size_t)G.fsize;
   const size_t nstate = (size_t)2 * (nc + 6 + (C.lsoil ? 1 : 0));
-  const size_t ndiff = diffusion ? (size_t)14 + nc + 3 * (nc + 1) : 0;  // the diffusion and surface fields of WorkT
+  const size_t ndiff = diffusion ? (size_t)14 + nc : 0;  // the diffusion and surface fields of WorkT
   const size_t nwork = (size_t)nc + 4 + 5 + 6 + 4 + 7 + 10 + 2 + ndiff;
   const size_t ncol = 13;  // 12 column-scratch fields and the cloud-water sink velocity
   const size_t wbytes = mixed ? sizeof(float) : sizeof(double);
@@ -810,11 +801,6 @@ int lgame_init(const lgame_dims *dims, const lgame_cfg *cfg, const lgame_grid_vi
       W.sfc = take();
       W.sfc2 = take();
       for (int jc = 0; jc < MAX_CONST; ++jc) W.mdt[jc] = jc < nc ? take() : nullptr;
-      for (int q = 0; q <= MAX_CONST; ++q) {
-        W.dfu[q] = q <= nc ? take() : nullptr;
-        W.dfv[q] = q <= nc ? take() : nullptr;
-        W.dfw[q] = q <= nc ? take() : nullptr;
-      }
     }
     for (int q = 0; q < 12; ++q) W.col[q] = col[q];
     W.vfall_cw = col[12];
@@ -1786,6 +1772,10 @@ int enqueue_group(lgame_ensemble *e, BatchGroup &g, int a_slot, int b_slot, int 
       batch_launch_scalar<R>(grd, blk, st, M, pf, n, a, g.moist, g.o3, C.ltemp_h || C.lmass_h);
       return;
     }
+    if (ph == PH_DIFF_FLUX) {
+      batch_launch_diff_col<R>(grd, blk, st, M, pf, n, a, g.moist, C.ltemp_h, C.lmass_h);
+      return;
+    }
     if (!batch_launch_step<R>(ph, grd, blk, st, M, pf, n, a) && !batch_launch_diff<R>(ph, grd, blk, st, M, pf, n, a))
       (void)batch_launch_solve<R>(ph, grd, blk, st, M, pf, n, a);
   };
@@ -1841,7 +1831,6 @@ int enqueue_group(lgame_ensemble *e, BatchGroup &g, int a_slot, int b_slot, int 
       launch(PH_VEC_TEND, a);
     if (rk == 1 && (C.ltemp_h || C.lmass_h)) {
       launch(PH_DIFF_FLUX, a);
-      launch(PH_DIFF_DIV, a);
     }
     if (g.o3 && rk == 2) {
       BatchArgs t = a;

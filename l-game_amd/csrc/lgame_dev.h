@@ -38,6 +38,10 @@ constexpr int MAX_CONST = 7;
 // soil layers the surface kernel holds in registers
 constexpr int MAX_SOIL = 16;
 
+// The columns (cells) of a 64-lane row of a column-marching kernel; the first and the last lane hold the
+// west and the east neighbour of its cells.
+constexpr int SCOL_CELLS = 62;
+
 // XCDs of the MI355X; blocks of a launch go to them round-robin.
 constexpr int N_XCD = 8;
 
@@ -115,11 +119,9 @@ struct WorkT {
   // kinematic viscosity, diag%viscosity), mom_x/_y/_z (diag%mom_diff_tend_*), tdh
   // (diag%temp_diff_heating) and mdt (diag%mass_diff_tendency).  Per step: zeta (relative
   // vorticity at the dual points), tke_next, kv (molecular plus vertical eddy viscosity of a
-  // cell), vdiv (visc times the horizontal divergence), vz (viscosity_dual times zeta) and the
-  // diffusive fluxes dfu, dfv, dfw of the temperature (index 0) and the densities (1..nc).
+  // cell), vdiv (visc times the horizontal divergence) and vz (viscosity_dual times zeta).
   // rsum is sum(rho(1:ncond+1)) of the old state, stored by k_temperature.
   Fld<R> tke, tke_next, visc, kv, vdiv, zeta, vz, mom_x, mom_y, mom_z, tdh, mdt[MAX_CONST], rsum;
-  Fld<R> dfu[MAX_CONST + 1], dfv[MAX_CONST + 1], dfw[MAX_CONST + 1];
   // surface turbulence: diag%roughness_length, roughness_velocity, monin_obukhov_length at
   // levels 1, 2, 3; surface heat: diag%scalar_flux_resistance, power_flux_density_sens_soil and
   // power_flux_density_sens_sea at levels 1, 2, 3 of sfc2

@@ -22,6 +22,38 @@ namespace lgame {
 
 __device__ __forceinline__ int wrapm(int i, int n) { return i == 1 ? n : i - 1; }
 
+// ---- several quotients with one denominator ----------------------------------------------------
+// a/b, correctly rounded as the operator's, from a reciprocal of b that is formed once.
+// FP64: y is 1/b rounded to nearest.  q = a*y is within two units in the last place; the residual
+// a - b*q is exact in one fused multiply-add, and a correction with y leaves less than one unit, after
+// which a second correction rounds as a/b does (P. Markstein, "Computation of elementary functions on
+// the IBM RISC System/6000 processor", IBM J. Res. Dev. 34, 1990).  Where the residual is not a number
+// (an infinite a or b), q itself is the operator's value.  (Below about 1e-290 the residual can
+// underflow and the last place may differ.)
+// FP32: the FP64 product is off by at most 2^-51 relative, and a quotient of two 24-bit numbers is never
+// within 2^-49 of the middle between two 24-bit numbers, so its rounding is that of a/b.
+// Five fused operations and a select (FP64) or a product between two conversions (FP32) take the place
+// of the operator's scaled Newton iteration of twelve, five of them at a quarter of the rate.
+template <class R>
+struct Inv;
+template <>
+struct Inv<double> {
+  double b, y;
+  __device__ __forceinline__ explicit Inv(double x) : b(x), y(1.0 / x) {}
+};
+template <>
+struct Inv<float> {
+  double y;
+  __device__ __forceinline__ explicit Inv(float x) : y(1.0 / (double)x) {}
+};
+__device__ __forceinline__ double operator/(double a, Inv<double> d) {
+  const double q = a * d.y;
+  const double q1 = __builtin_fma(__builtin_fma(-d.b, q, a), d.y, q);
+  const double q2 = __builtin_fma(__builtin_fma(-d.b, q1, a), d.y, q1);
+  return q2 == q2 ? q2 : q;
+}
+__device__ __forceinline__ float operator/(float a, Inv<float> d) { return (float)((double)a * d.y); }
+
 // ---- two x-adjacent points per thread -------------------------------------------------------
 // A stencil can be evaluated at the columns k and k+1 of one row at once (k odd, k+1 <= nx).  Its
 // values are then pairs: the loads of the own columns are single 2-element vector loads (aligned,
@@ -401,6 +433,52 @@ __device__ __forceinline__ VT<R, X> ke_point(const CtxT<R> &c, const StateDev &s
          LDG(c.g.ipw[3], ji, jk, jl) * v1 * v1 + LDG(c.g.ipw[4], ji, jk, jl) * w0 * w0 + LDG(c.g.ipw[5], ji, jk, jl) * w1 * w1;
 }
 
+// ---- column-marching kernels: 64 lanes of a row, 62 of them cells --------------------------------
+// the value of `x` at the next (down) or previous (up) lane of the wavefront
+// (as data-parallel moves of the vector unit: a shift of the whole wavefront by one lane; lane 63 gets no
+// next and lane 0 no previous value, they get 0)
+template <int CTRL>
+__device__ __forceinline__ int dpp(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+  return __int_as_float(dpp<CTRL>(__float_as_int(x)));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp(double x) {
+  return __hiloint2double(dpp<CTRL>(__double2hiint(x)), dpp<CTRL>(__double2loint(x)));
+}
+constexpr int WAVE_SHL1 = 0x130, WAVE_SHR1 = 0x138;
+template <class T>
+__device__ __forceinline__ T from_next_lane(T x) {
+  return dpp<WAVE_SHL1>(x);
+}
+template <class T>
+__device__ __forceinline__ T from_prev_lane(T x) {
+  return dpp<WAVE_SHR1>(x);
+}
+
+// this lane's place: row ji, lane column jk (0..nx+1 and beyond), the state column js (jk
+// wrapped), the metric column jkm (jk clamped to the stored u points), the wrapped rows jmr
+// (ji-1) and j1 (ji+1), and whether the lane's column is a cell of this row
+struct Lane {
+  int ji, jk, js, jkm, jmr, j1;
+  bool cell;
+};
+__device__ __forceinline__ Lane col_lane(const Geom &G, int tx, int ji) {
+  Lane p;
+  const int nx = G.nx, lane = (int)threadIdx.x;
+  p.ji = ji;
+  p.jk = tx * SCOL_CELLS + lane;  // lane 0: the west halo column
+  p.js = p.jk < 1 ? nx : (p.jk > nx ? 1 : p.jk);
+  p.jkm = p.jk < 1 ? 1 : (p.jk > nx + 1 ? nx + 1 : p.jk);
+  p.jmr = wrapm(ji, G.ny);
+  p.j1 = ji == G.ny ? 1 : ji + 1;
+  p.cell = lane >= 1 && lane <= SCOL_CELLS && p.jk <= nx;
+  return p;
+}
+
 // ---- thread -> grid point maps of the stencil kernels ---------------------------------------
 // Every kernel body takes its block's coordinates `bid` as an argument: from blockIdx when the
 // kernel runs for one domain, from an ensemble's work list when one launch covers several.
@@ -501,25 +579,11 @@ template <class V>
 struct VccGeo {
   V sx1, sy0, sx0, sy1, w0, w1, w2, w3;
 };
-template <class R, class X>
-__device__ __forceinline__ VccGeo<VT<R, X>> vcc_geo(const CtxT<R> &c, int ji, X jk, int l) {
-  const auto ke = east(jk);
-  return VccGeo<VT<R, X>>{LDG(c.g.slope_x, ji, ke, l), LDG(c.g.slope_y, ji, jk, l),     LDG(c.g.slope_x, ji, jk, l),
-                          LDG(c.g.slope_y, ji + 1, jk, l), LDG(c.g.ipw[0], ji, jk, l), LDG(c.g.ipw[1], ji, jk, l),
-                          LDG(c.g.ipw[2], ji, jk, l),      LDG(c.g.ipw[3], ji, jk, l)};
-}
-
 // a vector field at the four faces of cell (ji, jk): x at jk+1, y at ji, x at jk, y at ji+1
 template <class V>
 struct Faces {
   V e, n, w, s;
 };
-template <class R, class P, class X>
-__device__ __forceinline__ Faces<VT<R, X>> faces(P vx, P vy, const Geom &G, int ji, X jk, int l) {
-  return Faces<VT<R, X>>{cvt<R>(ldv(vx, G, ji, east(jk), l)), cvt<R>(ldv(vy, G, ji, jk, l)), cvt<R>(ldv(vx, G, ji, jk, l)),
-                         cvt<R>(ldv(vy, G, ji + 1, jk, l))};
-}
-
 // the element type of a value or a pair
 template <class V>
 struct ElemOf {

@@ -27,30 +27,12 @@ namespace lgame {
 
 namespace {
 
-// the value of `x` at the next (down) or previous (up) lane of the wavefront
-template <class T>
-__device__ __forceinline__ T from_next_lane(T x) {
-  return __shfl_down(x, 1, 64);
-}
-template <class T>
-__device__ __forceinline__ T from_prev_lane(T x) {
-  return __shfl_up(x, 1, 64);
-}
-
 // the constituents: the moist layout is fixed at 5 condensates, the gas and the vapour (lgame_init
 // accepts no other), the dry one is the gas alone
 template <bool TR>
 struct Cons {
   static constexpr int nc = TR ? 7 : 1, ncond = TR ? 5 : 0;
   static constexpr bool tracer(int q) { return TR && q != ncond; }
-};
-
-// this lane's place: row ji, lane column jk (0..nx+1 and beyond), the state column js (jk
-// wrapped), the metric column jkm (jk clamped to the stored u points), the wrapped rows jmr
-// (ji-1) and j1 (ji+1), and whether the lane's column is a cell of this row
-struct Lane {
-  int ji, jk, js, jkm, jmr, j1;
-  bool cell;
 };
 
 // the correction of one interface for the three flux kinds
@@ -284,16 +266,8 @@ __device__ __forceinline__ void b_scalar_col(const CtxT<R> &c, const StateDev &s
   const int k = b % N_XCD, s = b / N_XCD, q = n / N_XCD, rr = n % N_XCD;
   const int t = k * q + (k < rr ? k : rr) + s;
   const int tx = t % tx_n, ty = (t / tx_n) % ty_n, seg = t / (tx_n * ty_n);
-  Lane p;
-  p.ji = ty * (int)blockDim.y + (int)threadIdx.y + 1;
+  const Lane p = col_lane(G, tx, ty * (int)blockDim.y + (int)threadIdx.y + 1);
   if (p.ji > ny) return;  // a whole row (wavefront) at once
-  const int lane = (int)threadIdx.x;
-  p.jk = tx * SCOL_CELLS + lane;  // lane 0: the west halo column
-  p.js = p.jk < 1 ? nx : (p.jk > nx ? 1 : p.jk);
-  p.jkm = p.jk < 1 ? 1 : (p.jk > nx + 1 ? nx + 1 : p.jk);
-  p.jmr = wrapm(p.ji, ny);
-  p.j1 = p.ji == ny ? 1 : p.ji + 1;
-  p.cell = lane >= 1 && lane <= SCOL_CELLS && p.jk <= nx;
   // this segment's levels
   const int l0 = 1 + (nl * seg) / nseg, l1 = (nl * (seg + 1)) / nseg;
   const Corr<R> zero{R(0.0), R(0.0), R(0.0)};

@@ -27,10 +27,6 @@ template <class R> __global__ void k_diff_coef(const CtxT<R> c, const StateDev s
 template <class R> __global__ void k_diff_coef2(const CtxT<R> c, const StateDev s);  // nx even: two cells per thread
 template <class R> __global__ void k_diff_dual(const CtxT<R> c, const StateDev s);
 template <class R> __global__ void k_diff_mom(const CtxT<R> c, const StateDev s);
-template <class R> __global__ void k_diff_flux(const CtxT<R> c, const StateDev s);
-template <class R> __global__ void k_diff_flux2(const CtxT<R> c, const StateDev s);  // nx even: two cells per thread
-template <class R> __global__ void k_diff_div(const CtxT<R> c);
-template <class R> __global__ void k_diff_div2(const CtxT<R> c);  // nx even: two cells per thread
 template <class R> __global__ void k_sfc_turb(const CtxT<R> c, const StateDev s);
 template <class R> __global__ void k_pbl_wind(const CtxT<R> c, const StateDev s);
 template <class R> __global__ void k_surface(const CtxT<R> c, const StateDev old, const StateDev nw, int rk);
@@ -42,9 +38,10 @@ constexpr int BY = 4;
 
 // stencil kernels of the step, the index of their tile-table entry.  The mass fluxes and the
 // kinetic energy are formed in the potential-vorticity kernel, the kinetic-energy gradient in the
-// vorticity-flux kernel, the scalar fluxes in the scalar column kernel and the full theta_v of the
-// third-order theta where the gradient and edge kernels load it: KI_THETA_FILL, KI_MASS_FLUX, KI_KE,
-// KI_KE_GRAD and KI_SCALAR_FLUX keep their place in the table (and the C-ABI's order) unused.
+// vorticity-flux kernel, the scalar fluxes in the scalar column kernel, the divergence of the diffusive
+// fluxes in the diffusion column kernel (KI_DIFF_FLUX) and the full theta_v of the third-order theta
+// where the gradient and edge kernels load it: KI_THETA_FILL, KI_MASS_FLUX, KI_KE, KI_KE_GRAD,
+// KI_SCALAR_FLUX and KI_DIFF_DIV keep their place in the table (and the C-ABI's order) unused.
 enum KernelId {
   KI_TEMPERATURE, KI_THETA_FILL, KI_THETA_GRAD, KI_THETA_DIV, KI_THETA_EDGE, KI_PGRAD, KI_POT_VORT, KI_MASS_FLUX,
   KI_VORT_FLUX, KI_KE, KI_KE_GRAD, KI_DISSIPATION, KI_VEC_TEND, KI_SCALAR_FLUX, KI_SCALAR_DIV, KI_DIFF_ZETA,
@@ -64,7 +61,6 @@ struct Tiles {
 
 // The column-marching scalar_tend_expl (k_scalar_col): 64-lane rows of which 62 lanes are cells
 // and two the west and east halo; `rows` rows per block, the levels cut into `nseg` segments.
-constexpr int SCOL_CELLS = 62;
 // segments that give a domain about four wavefronts per SIMD of the MI355X (1024 SIMDs), with at
 // least four levels per segment
 inline int default_segments(const Geom &G) {
@@ -75,6 +71,9 @@ inline int default_segments(const Geom &G) {
 }
 template <class R>
 void launch_scalar_col(const CtxT<R> &c, const StateDev &ss, const StateDev &nw, int rk, int rows, int nseg, hipStream_t st);
+// the diffusive tendencies of the temperature and the densities, on the same launch geometry
+template <class R>
+void launch_diff_col(const CtxT<R> &c, const StateDev &s, int rows, int nseg, hipStream_t st);
 // Lanes per block of the column solvers.
 constexpr int BCOL = 64;
 // The vertical solver with a column's levels cut into segments held in registers (k_ver_seg): columns

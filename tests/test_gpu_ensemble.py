@@ -134,6 +134,31 @@ def test_batched_vertical_solver_with_members_of_different_height(layers):
         s.close()
 
 
+DIFF_SWITCHES = {"all": {}, "temperature": dict(lmass_diff_h=False, lmass_diff_v=False),
+                 "densities": dict(ltemp_diff_h=False, ltemp_diff_v=False), "horizontal": dict(ltemp_diff_v=False, lmass_diff_v=False)}
+
+
+@pytest.mark.parametrize("switches", list(DIFF_SWITCHES))
+@pytest.mark.parametrize("nx,nl,oro,moist,rows,seg", [(61, 16, 12, True, 1, 4), (62, 9, 8, False, 2, 2), (63, 6, 4, True, 4, 1),
+                                                      (125, 5, 1, False, 4, 1)])
+def test_diffusion_columns_match_oracle(nx, nl, oro, moist, rows, seg, switches):
+    """The scalar diffusion marches down 62-cell row tiles, cut into vertical segments: one partial
+    tile, full ones and a third, with flat and terrain-following layers, every set
+    of switches, bitwise against the oracle."""
+    cfg = dataclasses.replace(tiny_config(ny=5, nx=nx, n_layers=nl, moist=moist).set_diffusion(), n_oro_layers=oro,
+                              **DIFF_SWITCHES[switches])
+    g, st = make_case(cfg, cloud_frac=0.3 if moist else 0.0)
+    want = _oracle(cfg, g, st, 3)
+    s = Step(cfg, g)
+    s.set_tiles({k: rows for k in TILE_KERNELS})
+    s.segments = seg
+    s.start(st)
+    s.run(0, 3)
+    got = s.get_state(1)
+    s.close()
+    assert all(np.array_equal(got[k], want[k]) for k in want)
+
+
 def test_vertical_solver_default_passes_by_size():
     """One pass per column once the domain has as many 64-column wavefronts as the GPU has SIMDs."""
     for n, want in ((128, 3), (256, 1)):
