@@ -20,7 +20,7 @@ namespace lgame {
 // second substep's wind update alone (runs without momentum advection).  PH_VER_SEG takes the place of
 // PH_SOLVE_VER when ver_segments holds for every member.
 enum Phase : int {
-  PH_TEMPERATURE, PH_SFC_TURB, PH_THETA_GRAD, PH_THETA_DIV, PH_THETA_EDGE, PH_PGRAD, PH_POT_VORT,
+  PH_TEMPERATURE, PH_SFC_TURB, PH_THETA_DIV, PH_THETA_EDGE, PH_PGRAD, PH_POT_VORT,
   PH_VORT_FLUX, PH_DIFF_ZETA, PH_DIFF_COEF, PH_DIFF_DUAL, PH_DIFF_MOM, PH_PBL_WIND,
   PH_DISSIPATION, PH_VEC_TEND, PH_DIFF_FLUX, PH_SCALAR, PH_SURFACE, PH_SOLVE_VER, PH_SOLVE_GEN, PH_RAD,
   PH_VORT_FLUX_VT, PH_VER_SEG,
@@ -32,7 +32,6 @@ inline int phase_tile(int ph) {
   switch (ph) {
     case PH_TEMPERATURE: return KI_TEMPERATURE;
     case PH_SFC_TURB: case PH_PBL_WIND: case PH_SURFACE: case PH_DIFF_DUAL: return KI_DIFF_DUAL;
-    case PH_THETA_GRAD: return KI_THETA_GRAD;
     case PH_THETA_DIV: return KI_THETA_DIV;
     case PH_THETA_EDGE: return KI_THETA_EDGE;
     case PH_PGRAD: return KI_PGRAD;
@@ -78,13 +77,13 @@ __host__ __device__ inline void phase_grid(int ph, const Geom &G, int by, int se
   bool flat = false;  // a 1-D grid (tile_zfast kernels)
   gx = gy = gz = 0;
   switch (ph) {
-    case PH_TEMPERATURE: case PH_THETA_DIV: case PH_DIFF_DUAL: case PH_DISSIPATION: break;
+    case PH_TEMPERATURE: case PH_DIFF_DUAL: case PH_DISSIPATION: break;
     case PH_SFC_TURB: case PH_PBL_WIND: case PH_SURFACE: ez = 1; break;
-    case PH_THETA_GRAD: case PH_THETA_EDGE: case PH_VEC_TEND: ex = nx + 1; ey = ny + 1; break;
+    case PH_THETA_EDGE: case PH_VEC_TEND: ex = nx + 1; ey = ny + 1; break;
     case PH_PGRAD: case PH_VORT_FLUX: case PH_VORT_FLUX_VT: case PH_DIFF_COEF: case PH_DIFF_MOM: flat = true; break;
     case PH_POT_VORT: ez = nlev; flat = true; break;
     case PH_DIFF_ZETA: ex = nx + 1; ey = ny + 1; flat = true; break;
-    case PH_SCALAR: case PH_DIFF_FLUX: gx = ((nx + SCOL_CELLS - 1) / SCOL_CELLS) * ((ny + by - 1) / by) * seg; gy = gz = 1; return;
+    case PH_SCALAR: case PH_THETA_DIV: case PH_DIFF_FLUX: gx = ((nx + SCOL_CELLS - 1) / SCOL_CELLS) * ((ny + by - 1) / by) * seg; gy = gz = 1; return;
     case PH_SOLVE_VER: gx = col_waves(G); gy = gz = 1; return;
     case PH_VER_SEG: gx = vs_blocks_per_row(G.nx) * G.ny; gy = gz = 1; return;
     case PH_RAD: gx = (nx * ny + BCOL - 1) / BCOL; gy = gz = 1; return;
@@ -152,6 +151,9 @@ template <class R>
 void batch_launch_scalar(dim3 g, dim3 b, hipStream_t st, const MemberDev<R> *M, const int *prefix, int nm, const BatchArgs &a,
                          bool tr, bool o3, bool diff);
 
+// the theta column kernel, for a.nfield fields
+template <class R>
+void batch_launch_theta_col(dim3 g, dim3 b, hipStream_t st, const MemberDev<R> *M, const int *prefix, int nm, const BatchArgs &a);
 // the diffusion column kernel, with its moist, temperature and density variants chosen by tr, temp, mass
 template <class R>
 void batch_launch_diff_col(dim3 g, dim3 b, hipStream_t st, const MemberDev<R> *M, const int *prefix, int nm, const BatchArgs &a,

@@ -315,6 +315,11 @@ int enqueue_pchevi(const CtxT<R> &c, const StateDev &old, const StateDev &nw, in
     if (pk) prof->end(PROF_KERNEL0 + (KI));                                                \
   } while (0)
 
+  auto theta_div = [&](const StateDev &s, int nfield) {
+    if (pk) prof->begin(PROF_KERNEL0 + KI_THETA_DIV);
+    launch_theta_col(c, s, nfield, tiles.by[KI_THETA_DIV], tiles.seg, st);
+    if (pk) prof->end(PROF_KERNEL0 + KI_THETA_DIV);
+  };
   LG_LAUNCH(KI_TEMPERATURE, k_temperature, nx, ny, nl, c, old);
   // update_sfc_turb_quantities with state_old (mo_manage_pchevi.F90:52-54)
   if (c.C.lsfc_turb) LG_LAUNCH(KI_DIFF_DUAL, k_sfc_turb, nx, ny, 1, c, old);
@@ -330,8 +335,7 @@ int enqueue_pchevi(const CtxT<R> &c, const StateDev &old, const StateDev &nw, in
     if (rk == 1) {
       // manage_p_grad (mo_p_grad.F90:20-104); theta_v_adv_3rd_order of theta_v and theta_v_pert
       if (o3) {
-        LG_LAUNCH(KI_THETA_GRAD, k_theta_grad, nx + 1, ny + 1, nl, c, old, 2);
-        LG_LAUNCH(KI_THETA_DIV, k_theta_div, nx, ny, nl, c, 2);
+        theta_div(old, 2);
         LG_LAUNCH(KI_THETA_EDGE, k_theta_edge, nx + 1, ny + 1, nl, c, old, 2);
       }
     }
@@ -389,8 +393,7 @@ int enqueue_pchevi(const CtxT<R> &c, const StateDev &old, const StateDev &nw, in
     // scalar_tend_expl (mo_scalar_tend_expl.F90:24-181); at rk 1 the theta_v edge values of the
     // pressure gradient are reused (same state, same winds)
     if (o3 && rk == 2) {
-      LG_LAUNCH(KI_THETA_GRAD, k_theta_grad, nx + 1, ny + 1, nl, c, nw, 1);
-      LG_LAUNCH(KI_THETA_DIV, k_theta_div, nx, ny, nl, c, 1);
+      theta_div(nw, 1);
       LG_LAUNCH(KI_THETA_EDGE, k_theta_edge, nx + 1, ny + 1, nl, c, nw, 1);
     }
     if (pk) prof->begin(PROF_KERNEL0 + KI_SCALAR_DIV);
@@ -708,7 +711,7 @@ int lgame_init(const lgame_dims *dims, const lgame_cfg *cfg, const lgame_grid_vi
   const size_t fs = (size_t)G.fsize;
   const size_t nstate = (size_t)2 * (nc + 6 + (C.lsoil ? 1 : 0));
   const size_t ndiff = diffusion ? (size_t)14 + nc : 0;  // the diffusion and surface fields of WorkT
-  const size_t nwork = (size_t)nc + 4 + 5 + 6 + 4 + 7 + 10 + 2 + ndiff;
+  const size_t nwork = (size_t)nc + 4 + 5 + 6 + 4 + 7 + 6 + 2 + ndiff;
   const size_t ncol = 13;  // 12 column-scratch fields and the cloud-water sink velocity
   const size_t wbytes = mixed ? sizeof(float) : sizeof(double);
   h->slab_bytes = (nstate + NGRID + ncol) * fs * sizeof(double) + nwork * fs * wbytes + (mixed ? NGRID * fs * sizeof(float) : 0);
@@ -777,8 +780,6 @@ int lgame_init(const lgame_dims *dims, const lgame_cfg *cfg, const lgame_grid_vi
     W.w_ph = take();
     W.v_squared = take();
     for (int q = 0; q < 2; ++q) {
-      W.tgu[q] = take();
-      W.tgv[q] = take();
       W.tfd[q] = take();
       W.tu[q] = take();
       W.tv[q] = take();
@@ -1772,6 +1773,10 @@ int enqueue_group(lgame_ensemble *e, BatchGroup &g, int a_slot, int b_slot, int 
       batch_launch_scalar<R>(grd, blk, st, M, pf, n, a, g.moist, g.o3, C.ltemp_h || C.lmass_h);
       return;
     }
+    if (ph == PH_THETA_DIV) {
+      batch_launch_theta_col<R>(grd, blk, st, M, pf, n, a);
+      return;
+    }
     if (ph == PH_DIFF_FLUX) {
       batch_launch_diff_col<R>(grd, blk, st, M, pf, n, a, g.moist, C.ltemp_h, C.lmass_h);
       return;
@@ -1811,7 +1816,7 @@ int enqueue_group(lgame_ensemble *e, BatchGroup &g, int a_slot, int b_slot, int 
         BatchArgs t = a;
         t.state_slot = a_slot;
         t.nfield = 2;
-        for (int ph : {PH_THETA_GRAD, PH_THETA_DIV, PH_THETA_EDGE}) launch(ph, t);
+        for (int ph : {PH_THETA_DIV, PH_THETA_EDGE}) launch(ph, t);
       }
     }
     bool winds_done = false;
@@ -1836,7 +1841,7 @@ int enqueue_group(lgame_ensemble *e, BatchGroup &g, int a_slot, int b_slot, int 
       BatchArgs t = a;
       t.state_slot = b_slot;
       t.nfield = 1;
-      for (int ph : {PH_THETA_GRAD, PH_THETA_DIV, PH_THETA_EDGE}) launch(ph, t);
+      for (int ph : {PH_THETA_DIV, PH_THETA_EDGE}) launch(ph, t);
     }
     launch(PH_SCALAR, a);
     if (C.lsoil || C.lsens) launch(PH_SURFACE, a);

@@ -340,7 +340,145 @@ const bool told = tr && rk == 2;
 template void launch_scalar_col<double>(const CtxT<double> &, const StateDev &, const StateDev &, int, int, int, hipStream_t);
 template void launch_scalar_col<float>(const CtxT<float> &, const StateDev &, const StateDev &, int, int, int, hipStream_t);
 
-// ---- the same kernel over a group of domains (one launch) --------------------------------------
+// ---------------------------------------------------------------------------------------------
+// The divergence of the horizontal theta gradient of theta_v_adv_3rd_order (mo_multiplications.F90:
+// 116-204), div_h of grad_hor, marching down the columns on the launch geometry of k_scalar_col (and as
+// k_diff_col, with unit coefficients): a lane forms the gradients at its west, north and south face of a
+// layer and finishes the cell above, which only waited for this layer's contravariant correction.
+// As a gradient kernel and a divergence kernel the gradients went through memory (four fields at the
+// first substep) and the metrics of three layers were loaded for every cell; both kernels were bound by
+// their load instructions.
+// FP64 161x129x47, us: the two kernels before 113 (mean of a step's two substeps) -> 48 (51 with two fields,
+// 45 with one); 201x3x40: 13.3 -> 12.4.
+// The gradients at column nx+1 and row ny+1 take the covariant part and the remap of column 1 and
+// row 1 and the slope stored there (grad_hor_x/_y).
+// NF: 2 fields, the full theta_v and its perturbation, or the first alone
+// ---------------------------------------------------------------------------------------------
+template <class R>
+struct ThetaField {
+  R c, n, s, vc, vn, vs, P, hh, I;  // as DiffField of k_diff_col
+};
+template <class R, int NF>
+__device__ __forceinline__ void b_theta_col(const CtxT<R> &c, const StateDev &st, int nseg, const Bid bid) {
+  const Geom &G = c.G;
+  const int nx = G.nx, ny = G.ny, nl = G.nl, nflat = G.nflat;
+  const int tx_n = (nx + SCOL_CELLS - 1) / SCOL_CELLS, ty_n = (ny + (int)blockDim.y - 1) / (int)blockDim.y;
+  const int nb = tx_n * ty_n * nseg, b = bid.x;
+  const int xk = b % N_XCD, xs = b / N_XCD, xq = nb / N_XCD, xr = nb % N_XCD;
+  const int t = xk * xq + (xk < xr ? xk : xr) + xs;
+  const int tx = t % tx_n, ty = (t / tx_n) % ty_n, seg = t / (tx_n * ty_n);
+  const Lane p = col_lane(G, tx, ty * (int)blockDim.y + (int)threadIdx.y + 1);
+  if (p.ji > ny) return;  // a whole row (wavefront) at once
+  const int l0 = 1 + (nl * seg) / nseg, l1 = (nl * (seg + 1)) / nseg;  // this segment's cells
+  const Fld<const double> pert = st.theta_v_pert;
+  // theta at a point: the full theta_v (field 0), its perturbation (field 1)
+  auto fld = [&](ix_t i, R (&v)[NF]) {
+    const R tp = R(pert[i]);
+    v[0] = c.g.theta_v_bg[i] + tp;
+    if (NF > 1) v[NF - 1] = tp;
+  };
+  const int m0 = l0 > 1 ? l0 - 1 : 1;  // the layer above the segment gives its correction terms
+  ThetaField<R> F[NF];
+  {
+    const ix_t iC = LG_IX(G, p.ji, p.js, m0), iN = LG_IX(G, p.jmr, p.js, m0), iS = LG_IX(G, p.j1, p.js, m0);
+    const ix_t dl = m0 > 1 ? (ix_t)G.lvl : 0;  // the interface above layer m0 (zero gradient at the top)
+    const R dzc = c.g.dz[iC], dzn = c.g.dz[iN], dzs = c.g.dz[iS];
+    R vc[NF], vn[NF], vs[NF], uc[NF], un[NF], us[NF];
+    fld(iC, vc);
+    fld(iN, vn);
+    fld(iS, vs);
+    fld(iC - dl, uc);
+    fld(iN - dl, un);
+    fld(iS - dl, us);
+#pragma unroll
+    for (int q = 0; q < NF; ++q) {
+      ThetaField<R> &f = F[q];
+      f.c = vc[q];
+      f.n = vn[q];
+      f.s = vs[q];
+      f.vc = m0 > 1 ? (uc[q] - vc[q]) / dzc : R(0.0);
+      f.vn = m0 > 1 ? (un[q] - vn[q]) / dzn : R(0.0);
+      f.vs = m0 > 1 ? (us[q] - vs[q]) / dzs : R(0.0);
+      f.P = f.hh = f.I = R(0.0);
+    }
+  }
+  R az_up = R(0.0);  // upper interface area and volume of the unfinished cell
+  Inv<R> V_up(R(1.0));
+  for (int m = m0; m <= l1 + 1; ++m) {  // (at m = n_layers+1 only the lowest cell is finished)
+    const bool terr = m > nflat;
+    const int ml = m < nl ? m : nl;  // (below the lowest layer, its own values once more)
+    const ix_t iC = LG_IX(G, p.ji, p.js, ml), iN = LG_IX(G, p.jmr, p.js, ml), iS = LG_IX(G, p.j1, p.js, ml);
+    const ix_t iM = LG_IX(G, p.ji, p.jkm, ml), iMs = LG_IX(G, p.ji + 1, p.jkm, ml);
+    const ix_t dl = ml < nl ? (ix_t)G.lvl : 0;
+    // all loads of the layer, issued before any is used
+    R nc[NF], nn[NF], ns[NF];
+    fld(iC + dl, nc);
+    fld(iN + dl, nn);
+    fld(iS + dl, ns);
+    const R dx_ = c.g.dx[iC], dyn_ = c.g.dy[iC], dys_ = c.g.dy[iS];
+    const R dzc_ = c.g.dz[iC + dl], dzn_ = c.g.dz[iN + dl], dzs_ = c.g.dz[iS + dl];
+    const R p4c = c.g.ipw[4][iC], p4n = c.g.ipw[4][iN], p4s = c.g.ipw[4][iS];
+    const R p5c = c.g.ipw[5][iC], p5n = c.g.ipw[5][iN], p5s = c.g.ipw[5][iS];
+    const R sxm = c.g.slope_x[iM], sym = c.g.slope_y[iM], syms = c.g.slope_y[iMs];
+    const R ax0 = c.g.area_x[iM], ay0 = c.g.area_y[iM], ay1 = c.g.area_y[iMs];
+    const R az = c.g.area_z[iC], vol = c.g.volume[iC];
+    const R w0 = c.g.ipw[0][iM], w1 = c.g.ipw[1][iM], w2 = c.g.ipw[2][iM], w3 = c.g.ipw[3][iM];
+    __builtin_amdgcn_sched_barrier(0);
+    const Inv<R> dx(dx_), dyn(dyn_), dys(dys_), dzc(dzc_), dzn(dzn_), dzs(dzs_);
+    const VccGeo<R> geo{from_next_lane(sxm), sym, sxm, syms, w0, w1, w2, w3};
+    const R ax1 = from_next_lane(ax0), p4w = from_prev_lane(p4c), p5w = from_prev_lane(p5c);
+    // the areas of the interfaces of the cell above that carry a contravariant correction and the slopes
+    // of the terrain-following layers, zero for the others (no branches below)
+    const int jl = m - 1;
+    const R az0 = jl > nflat ? az_up : R(0.0), az1 = jl >= nflat && jl < nl ? az : R(0.0);
+    const R sx = terr ? sxm : R(0.0), syn = terr ? sym : R(0.0), sys = terr ? syms : R(0.0);
+    const bool st_cell = p.cell && m > l0;
+    const ix_t iF = LG_IX(G, p.ji, p.js, m > 1 ? m - 1 : 1);
+#pragma unroll
+    for (int q = 0; q < NF; ++q) {
+      ThetaField<R> &f = F[q];
+      const R vc1 = (f.c - nc[q]) / dzc, vn1 = (f.n - nn[q]) / dzn, vs1 = (f.s - ns[q]) / dzs;
+      const R w = from_prev_lane(f.c), vw = from_prev_lane(f.vc), vw1 = from_prev_lane(vc1);
+      // grad_hor with remap_ver2hor_x/_y, mo_averaging.F90:56-136
+      const R gx = (f.c - w) / dx - sx * (R(0.5) * (p4w * vw + p4c * f.vc + p5w * vw1 + p5c * vc1));
+      const R gn = (f.n - f.c) / dyn - syn * (R(0.5) * (p4n * f.vn + p4c * f.vc + p5n * vn1 + p5c * vc1));
+      const R gs = (f.c - f.s) / dys - sys * (R(0.5) * (p4c * f.vc + p4s * f.vs + p5c * vc1 + p5s * vs1));
+      const Faces<R> fc{from_next_lane(gx), gn, gx, gs};
+      const R I = vcc_sub(f.P, geo, fc);
+      const R d = (f.hh + (f.I * az0 - I * az1)) / V_up;
+      if (st_cell) c.w.tfd[q][iF] = d;
+      f.hh = fc.e * ax1 + fc.n * ay0 - fc.w * ax0 - fc.s * ay1;
+      f.P = vcc_sub(R(0.0), geo, fc);
+      if (m <= nflat) f.P = R(0.0);  // interface nflat+1 has no terms of the layer above it
+      f.I = I;
+      f.c = nc[q];
+      f.n = nn[q];
+      f.s = ns[q];
+      f.vc = vc1;
+      f.vn = vn1;
+      f.vs = vs1;
+    }
+    az_up = az;
+    V_up = Inv<R>(vol);
+  }
+}
+template <class R, int NF>
+__global__ void __launch_bounds__(BX * 4) k_theta_col(const CtxT<R> c, const StateDev s, int nseg) {
+  b_theta_col<R, NF>(c, s, nseg, bid_here());
+}
+template <class R>
+void launch_theta_col(const CtxT<R> &c, const StateDev &s, int nfield, int rows, int nseg, hipStream_t st) {
+  const int tx_n = (c.G.nx + SCOL_CELLS - 1) / SCOL_CELLS, ty_n = (c.G.ny + rows - 1) / rows;
+  const dim3 blk(BX, rows, 1), grd((unsigned)(tx_n * ty_n * nseg));
+  if (nfield == 2)
+    hipLaunchKernelGGL((k_theta_col<R, 2>), grd, blk, 0, st, c, s, nseg);
+  else
+    hipLaunchKernelGGL((k_theta_col<R, 1>), grd, blk, 0, st, c, s, nseg);
+}
+template void launch_theta_col<double>(const CtxT<double> &, const StateDev &, int, int, int, hipStream_t);
+template void launch_theta_col<float>(const CtxT<float> &, const StateDev &, int, int, int, hipStream_t);
+
+// ---- the same kernels over a group of domains (one launch) --------------------------------------
 template <class R, bool TR, bool O3, bool DIFF, bool TOLD>
 __global__ void __launch_bounds__(BX * 4)
     kb_scalar_col(const MemberDev<R> *__restrict__ M, const int *__restrict__ prefix, int nm, const BatchArgs a) {
@@ -362,5 +500,22 @@ template void batch_launch_scalar<double>(dim3, dim3, hipStream_t, const MemberD
                                           bool, bool, bool);
 template void batch_launch_scalar<float>(dim3, dim3, hipStream_t, const MemberDev<float> *, const int *, int, const BatchArgs &,
                                          bool, bool, bool);
+
+template <class R, int NF>
+__global__ void __launch_bounds__(BX * 4)
+    kb_theta_col(const MemberDev<R> *__restrict__ M, const int *__restrict__ prefix, int nm, const BatchArgs a) {
+  Bid bid;
+  const MemberDev<R> &d = batch_block(M, prefix, nm, PH_THETA_DIV, bid);
+  b_theta_col<R, NF>(d.c, d.s[a.state_slot], d.seg, bid);
+}
+template <class R>
+void batch_launch_theta_col(dim3 g, dim3 b, hipStream_t st, const MemberDev<R> *M, const int *prefix, int nm, const BatchArgs &a) {
+  if (a.nfield == 2)
+    hipLaunchKernelGGL((kb_theta_col<R, 2>), g, b, 0, st, M, prefix, nm, a);
+  else
+    hipLaunchKernelGGL((kb_theta_col<R, 1>), g, b, 0, st, M, prefix, nm, a);
+}
+template void batch_launch_theta_col<double>(dim3, dim3, hipStream_t, const MemberDev<double> *, const int *, int, const BatchArgs &);
+template void batch_launch_theta_col<float>(dim3, dim3, hipStream_t, const MemberDev<float> *, const int *, int, const BatchArgs &);
 
 }  // namespace lgame

@@ -7,8 +7,6 @@
 namespace lgame {
 
 template <class R> __global__ void k_temperature(const CtxT<R> c, const StateDev s);
-template <class R> __global__ void k_theta_grad(const CtxT<R> c, const StateDev s, int nfield);
-template <class R> __global__ void k_theta_div(const CtxT<R> c, int nfield);
 template <class R> __global__ void k_theta_edge(const CtxT<R> c, const StateDev s, int nfield);
 // the potential vorticity, the mass fluxes and (with_ke) the kinetic energy
 template <class R> __global__ void k_pot_vort(const CtxT<R> c, const StateDev s, int with_ke);
@@ -40,8 +38,8 @@ constexpr int BY = 4;
 // kinetic energy are formed in the potential-vorticity kernel, the kinetic-energy gradient in the
 // vorticity-flux kernel, the scalar fluxes in the scalar column kernel, the divergence of the diffusive
 // fluxes in the diffusion column kernel (KI_DIFF_FLUX) and the full theta_v of the third-order theta
-// where the gradient and edge kernels load it: KI_THETA_FILL, KI_MASS_FLUX, KI_KE, KI_KE_GRAD,
-// KI_SCALAR_FLUX and KI_DIFF_DIV keep their place in the table (and the C-ABI's order) unused.
+// and its gradient in the theta column kernel (KI_THETA_DIV): KI_THETA_FILL, KI_THETA_GRAD, KI_MASS_FLUX,
+// KI_KE, KI_KE_GRAD, KI_SCALAR_FLUX and KI_DIFF_DIV keep their place in the table (and the C-ABI's order) unused.
 enum KernelId {
   KI_TEMPERATURE, KI_THETA_FILL, KI_THETA_GRAD, KI_THETA_DIV, KI_THETA_EDGE, KI_PGRAD, KI_POT_VORT, KI_MASS_FLUX,
   KI_VORT_FLUX, KI_KE, KI_KE_GRAD, KI_DISSIPATION, KI_VEC_TEND, KI_SCALAR_FLUX, KI_SCALAR_DIV, KI_DIFF_ZETA,
@@ -71,6 +69,9 @@ inline int default_segments(const Geom &G) {
 }
 template <class R>
 void launch_scalar_col(const CtxT<R> &c, const StateDev &ss, const StateDev &nw, int rk, int rows, int nseg, hipStream_t st);
+// the divergence of the theta gradient of theta_v_adv_3rd_order, on the same launch geometry
+template <class R>
+void launch_theta_col(const CtxT<R> &c, const StateDev &s, int nfield, int rows, int nseg, hipStream_t st);
 // the diffusive tendencies of the temperature and the densities, on the same launch geometry
 template <class R>
 void launch_diff_col(const CtxT<R> &c, const StateDev &s, int rows, int nseg, hipStream_t st);

@@ -76,44 +76,11 @@ __global__ void __launch_bounds__(BX * BY) k_temperature(const CtxT<R> c, const 
 }
 
 // ---------------------------------------------------------------------------------------------
-// theta_v_adv_3rd_order, mo_multiplications.F90:116-204, in three passes.
+// theta_v_adv_3rd_order, mo_multiplications.F90:116-204: the divergence of the gradient of theta
+// (k_theta_col), then the edge values.
 // field f: 0 = full theta_v (theta_v_bg + theta_v_pert), 1 = theta_v_pert.
 // ---------------------------------------------------------------------------------------------
-// pass 1a: scalar_placeholder = theta_v_bg + theta_v_pert (f=0) or theta_v_pert (f=1)
-// pass 1: u,v_placeholder = grad_hor(theta) with its grad_vert inline, theta being the full
-// theta_v of state s (field 0) or its theta_v_pert (field 1), formed at every load
-template <class R>
-__device__ __forceinline__ void b_theta_grad(const CtxT<R> &c, const StateDev &s, int nfield, const Bid bid) {
-  KIDX;
-  const int nx = c.G.nx, ny = c.G.ny;
-  if (jk > nx + 1 || ji > ny + 1 || jl > c.G.nl) return;
-  const ThetaFull<R> full{c.g.theta_v_bg, Fld<const double>(s.theta_v_pert)};
-  const Fld<const double> pert = s.theta_v_pert;
-  if (ji <= ny) AT(c.w.tgu[0], ji, jk, jl) = grad_hor_x(c, full, ji, jk, jl);
-  if (jk <= nx) AT(c.w.tgv[0], ji, jk, jl) = grad_hor_y(c, full, ji, jk, jl);
-  if (nfield > 1) {
-    if (ji <= ny) AT(c.w.tgu[1], ji, jk, jl) = grad_hor_x(c, pert, ji, jk, jl);
-    if (jk <= nx) AT(c.w.tgv[1], ji, jk, jl) = grad_hor_y(c, pert, ji, jk, jl);
-  }
-}
-template <class R>
-__global__ void __launch_bounds__(BX * BY) k_theta_grad(const CtxT<R> c, const StateDev s, int nfield) {
-  b_theta_grad(c, s, nfield, bid_here());
-}
-
-// pass 2: flux_density_div = div_h(u_placeholder, v_placeholder)
-template <class R>
-__device__ __forceinline__ void b_theta_div(const CtxT<R> &c, int nfield, const Bid bid) {
-  KIDX;
-  if (jk > c.G.nx || ji > c.G.ny || jl > c.G.nl) return;
-  for (int f = 0; f < nfield; ++f) AT(c.w.tfd[f], ji, jk, jl) = div_h(c, c.w.tgu[f], c.w.tgv[f], ji, jk, jl);
-}
-template <class R>
-__global__ void __launch_bounds__(BX * BY) k_theta_div(const CtxT<R> c, int nfield) {
-  b_theta_div(c, nfield, bid_here());
-}
-
-// pass 3: upwind-corrected edge values; the upwind direction comes from the given winds
+// upwind-corrected edge values; the upwind direction comes from the given winds
 template <class R>
 __device__ __forceinline__ void b_theta_edge(const CtxT<R> &c, const StateDev &s, int nfield, const Bid bid) {
   KIDX;
@@ -835,8 +802,6 @@ __global__ void __launch_bounds__(BX * BY) k_vort_flux_vt(const CtxT<R> c, const
 // The plain form (FP64 stencils) and the mixed form (FP32 stencils).
 #define LG_INSTANTIATE(R)                                                                                  \
   template __global__ void k_temperature<R>(const CtxT<R>, const StateDev);                              \
-  template __global__ void k_theta_grad<R>(const CtxT<R>, const StateDev, int);                          \
-  template __global__ void k_theta_div<R>(const CtxT<R>, int);                                           \
   template __global__ void k_theta_edge<R>(const CtxT<R>, const StateDev, int);                          \
   template __global__ void k_pot_vort<R>(const CtxT<R>, const StateDev, int);                            \
   template __global__ void k_pot_vort2<R>(const CtxT<R>, const StateDev, int);                           \
@@ -852,8 +817,6 @@ LG_INSTANTIATE(float)
 
 // ---- the same kernels over a group of domains (one launch per phase) ------------------------
 LG_BATCH_KERNEL(temperature, BX * BY, PH_TEMPERATURE, b_temperature(d.c, d.s[a.old_slot], bid))
-LG_BATCH_KERNEL(theta_grad, BX * BY, PH_THETA_GRAD, b_theta_grad(d.c, d.s[a.state_slot], a.nfield, bid))
-LG_BATCH_KERNEL(theta_div, BX * BY, PH_THETA_DIV, b_theta_div(d.c, a.nfield, bid))
 LG_BATCH_KERNEL(theta_edge, BX * BY, PH_THETA_EDGE, b_theta_edge(d.c, d.s[a.state_slot], a.nfield, bid))
 LG_BATCH_KERNEL(pgrad, BX * BY, PH_PGRAD, b_pgrad_vt(d.c, d.s[a.old_slot], d.s[a.new_slot], a.lfirst, bid))
 LG_BATCH_KERNEL(pot_vort, BX * BY, PH_POT_VORT, b_pot_vort(d.c, d.s[a.state_slot], a.ke, bid))
@@ -870,8 +833,6 @@ bool batch_launch_step(int ph, dim3 g, dim3 b, hipStream_t st, const MemberDev<R
     return true;
   switch (ph) {
     LG_B(PH_TEMPERATURE, kb_temperature)
-    LG_B(PH_THETA_GRAD, kb_theta_grad)
-    LG_B(PH_THETA_DIV, kb_theta_div)
     LG_B(PH_THETA_EDGE, kb_theta_edge)
     LG_B(PH_PGRAD, kb_pgrad)
     LG_B(PH_POT_VORT, kb_pot_vort)

@@ -159,6 +159,24 @@ def test_diffusion_columns_match_oracle(nx, nl, oro, moist, rows, seg, switches)
     assert all(np.array_equal(got[k], want[k]) for k in want)
 
 
+@pytest.mark.parametrize("ny,nx,nl,oro,moist,rows,seg", [(5, 61, 16, 12, True, 1, 4), (6, 62, 9, 8, False, 2, 2), (5, 63, 6, 4, True, 4, 1),
+                                                         (3, 125, 5, 1, False, 4, 1)])
+def test_third_order_theta_columns_match_oracle(ny, nx, nl, oro, moist, rows, seg):
+    """The divergence of the theta gradient marches down 62-cell row tiles in vertical segments: one partial
+    tile, full ones and a third, the fewest rows, flat and terrain-following layers, bitwise against the oracle."""
+    cfg = dataclasses.replace(tiny_config(ny=ny, nx=nx, n_layers=nl, moist=moist, order=3), n_oro_layers=oro)
+    g, st = make_case(cfg, cloud_frac=0.3 if moist else 0.0)
+    want = _oracle(cfg, g, st, 3)
+    s = Step(cfg, g)
+    s.set_tiles({k: rows for k in TILE_KERNELS})
+    s.segments = seg
+    s.start(st)
+    s.run(0, 3)
+    got = s.get_state(1)
+    s.close()
+    assert all(np.array_equal(got[k], want[k]) for k in want)
+
+
 def test_vertical_solver_default_passes_by_size():
     """One pass per column once the domain has as many 64-column wavefronts as the GPU has SIMDs."""
     for n, want in ((128, 3), (256, 1)):
