@@ -407,8 +407,7 @@ int enqueue_pchevi(const CtxT<R> &c, const StateDev &old, const StateDev &nw, in
     if (prof) prof->end(0);
     if (c.G.nc > 1) {
       if (prof) prof->begin(1);
-      const dim3 g_gen((unsigned)((col_waves(c.G) + GEN_GROUPS - 1) / GEN_GROUPS));
-      hipLaunchKernelGGL(k_solve_gen<R>, g_gen, dim3(BCOL, NTR * GEN_GROUPS), 0, st, c, old, nw, rk);
+      launch_solve_gen(c, old, nw, rk, st);
       if (prof) prof->end(1);
     }
   }
@@ -1765,6 +1764,8 @@ int enqueue_group(lgame_ensemble *e, BatchGroup &g, int a_slot, int b_slot, int 
       blk = dim3(BCOL);
     else if (ph == PH_VER_SEG)
       blk = dim3(VS_THREADS);
+    else if (ph == PH_GEN_REG)
+      blk = dim3(BCOL, GR_WAVES);
     else if (ph == PH_SOLVE_GEN)
       blk = dim3(BCOL, NTR * GEN_GROUPS);
     else
@@ -1846,7 +1847,8 @@ int enqueue_group(lgame_ensemble *e, BatchGroup &g, int a_slot, int b_slot, int 
     launch(PH_SCALAR, a);
     if (C.lsoil || C.lsens) launch(PH_SURFACE, a);
     launch(ver_segments(g.nl_max) ? PH_VER_SEG : PH_SOLVE_VER, a);
-    if (g.moist) launch(PH_SOLVE_GEN, a);
+    if (g.moist && g.total[PH_GEN_REG]) launch(PH_GEN_REG, a);
+    if (g.moist && g.total[PH_SOLVE_GEN]) launch(PH_SOLVE_GEN, a);
   }
   ECHK(e, hipGetLastError());
   return 0;

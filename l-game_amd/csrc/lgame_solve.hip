@@ -768,6 +768,7 @@ __device__ __forceinline__ double c_p_water_sel(double temperature) {
 // inputs of layer l and of the interface below it (l+1)
 struct GenIn {
   double tr, wo, wn, az, Vb, ro_b, tif, vcw;  // vcw: cloud-water sink velocity of layer l+1
+  double qb, ct;                              // itw*dt/V of layer l+1; c_p times temperature there
 };
 
 // values carried from one layer to the next: the fluxes through the interface above, the
@@ -802,12 +803,8 @@ __device__ __forceinline__ GenRow gen_row(const GenIn &cur, GenCarry &s, double 
     fr = cur.az * fr;
     const double dens = fr >= 0.0 ? cur.ro_b : s.ro_cur;
     fr = dens * fr;
-    if (HEAT && cond) {
-      const double tif = cur.tif;
-      const double cp = CP == CP_ICE ? c_p_ice(tif) : c_p_water_sel(tif);
-      fe = cp * tif * fr;
-    }
-    q_b = itw * dt / cur.Vb;  // itw*dt/V of the layer below, also its q
+    if (HEAT && cond) fe = cur.ct * fr;
+    q_b = cur.qb;  // also the q of the layer below
   }
   const double q = s.q;
   GenRow w;
@@ -904,6 +901,7 @@ __device__ __forceinline__ void gen_sweep(const CtxT<R> &c, const StateDev &old,
     g.ro_b = ro[iw];
     g.tif = (HEAT && cond) ? (double)c.w.temperature[iw] : 0.0;  // temperature of layer l+1
     g.vcw = VF == VF_LIQUID ? c.w.vfall_cw[iw] : 0.0;
+    g.qb = g.ct = 0.0;
     return g;
   };
   const double az_sfc = AT(c.g64.area_z, ji, jk, nl + 1);
@@ -915,6 +913,11 @@ __device__ __forceinline__ void gen_sweep(const CtxT<R> &c, const StateDev &old,
   double V = c.g64.volume[LG_IX(c.G, ji, jk, 1)];
   s.q = 0.5 * dt / V;
   s.vcw_lo = VF == VF_LIQUID ? AT(c.w.vfall_cw, ji, jk, 1) : 0.0;
+  auto derive = [&](GenIn g) {
+    g.qb = 0.5 * dt / g.Vb;
+    if (HEAT && cond) g.ct = (CP == CP_ICE ? c_p_ice(g.tif) : c_p_water_sel(g.tif)) * g.tif;
+    return g;
+  };
   // heating terms of layer l go to ring slot (l-1) % GEN_RING
   auto put_heat = [&](const GenRow &w, int l) {
     if (HEAT && cond) sh.a[grp][(l - 1) % GEN_RING][t][lane] = w.ha;
@@ -936,7 +939,7 @@ __device__ __forceinline__ void gen_sweep(const CtxT<R> &c, const StateDev &old,
   };
   // two input buffers for odd and even layers, each refilled two layers ahead once used
   GenIn in_a = load(1), in_b = load(2);
-  GenRow row = gen_row<VF, CP, HEAT, POS_TOP>(in_a, s, vf_const, dt, V, az_sfc, t_sfc, hb_on, 1, nl);
+  GenRow row = gen_row<VF, CP, HEAT, POS_TOP>(derive(in_a), s, vf_const, dt, V, az_sfc, t_sfc, hb_on, 1, nl);
   V = in_a.Vb;
   put_heat(row, 1);
   in_a = load(3);  // n_layers >= 3
@@ -949,13 +952,13 @@ __device__ __forceinline__ void gen_sweep(const CtxT<R> &c, const StateDev &old,
         // (past the bottom the refill reloads layer nl, which is then never used)
         const int lf = l + 2 <= nl ? l + 2 : nl;
         if (l & 1) {
-          nxt = gen_row<VF, CP, HEAT, POS_MID>(in_a, s, vf_const, dt, V, az_sfc, t_sfc, hb_on, l, nl);
+          nxt = gen_row<VF, CP, HEAT, POS_MID>(derive(in_a), s, vf_const, dt, V, az_sfc, t_sfc, hb_on, l, nl);
           V = in_a.Vb;
           eliminate(row, jl);
           put_heat(nxt, l);
           in_a = load(lf);
         } else {
-          nxt = gen_row<VF, CP, HEAT, POS_MID>(in_b, s, vf_const, dt, V, az_sfc, t_sfc, hb_on, l, nl);
+          nxt = gen_row<VF, CP, HEAT, POS_MID>(derive(in_b), s, vf_const, dt, V, az_sfc, t_sfc, hb_on, l, nl);
           V = in_b.Vb;
           eliminate(row, jl);
           put_heat(nxt, l);
@@ -1099,10 +1102,316 @@ __global__ void __launch_bounds__(BCOL * NTR * GEN_GROUPS) k_solve_gen(const Ctx
   b_solve_gen(c, old, nw, rk, bid_here());
 }
 
+// ---- the same solve with the eliminated coefficients in registers and LDS ------------------------
+// The sweep and the back substitution of gen_sweep and gen_back on blocks of 64 columns.  r' of a column's
+// levels stays in register vectors (indexed by the level, which is uniform over a wavefront), e' of the four
+// tracers that have their own in LDS, so nothing goes through memory between the two.  LDS then holds one
+// block per CU, and what hides the latency is in the block: a seventh wavefront loads the winds and metrics
+// that the six tracers share four levels ahead, forms from them what does not depend on the tracer (itw*dt/V,
+// c_p T of ice and water) once instead of six times and leaves it in a ring of 2 KX levels; it also adds
+// up the sediment heating.  The tracer wavefronts load only their density and tendency, four levels ahead.
+// One barrier per KX levels: behind it the tracers read levels of the ring while the next KX are written,
+// and leave heating terms while those of the previous KX are added up.  KX is 4, or 2 with the heating, where
+// the ring holds more.
+// Bound by memory traffic (the scratch was 160 of 350 B per tracer column and level): us per launch at the
+// predictor and the corrector, k_solve_gen -> here: 512x512x60 FP64 1240, 1030 -> 880, 718 (4.5 TB/s), mixed
+// 1190, 990 -> 851, 703; 257x193x55 FP64 240 -> 203, 162.  Without the seventh wavefront (each tracer loading
+// everything, two levels ahead) it was bound by latency: 1517, 991.
+typedef double GenVec __attribute__((ext_vector_type(GR_PART)));
+enum { GS_WO, GS_WN, GS_AZ, GS_V, GS_QB, GS_CI, GS_CW };  // what the ring holds of a level: ... c_p T of ice, of water
+
+// One tracer.  stage: the ring, ep_col: e' of level 1 (levels BCOL apart), all at this lane
+template <class R, int VF, int CP, bool HEAT, bool OWN_EP>
+struct GenTracer {
+  static constexpr bool COND = CP != CP_NONE;
+  static constexpr int KX = gr_k(HEAT), NS = gr_fields(HEAT);
+  struct In {
+    R tr;  // converted where it is used, so that nothing waits for the load here
+    double ro_b, vcw;
+  };
+  const CtxT<R> &c;
+  const double *stage;
+  double *ha, *hb, *ep_col;
+  const Fld<const double> ro;
+  const Fld<const R> trd;
+  const int t, ji, jk, nl;
+  const double dt, vf_const, az_sfc, t_sfc;
+  const bool hb_on;
+  GenCarry s;
+  GenRow row;
+  double V, ep, rp, cprev;
+  GenVec r[GR_PARTS];
+  In in[4];
+
+  __device__ __forceinline__ In load(int l) const {
+    In g;
+    g.tr = trd[LG_IX(c.G, ji, jk, l)];
+    const ix_t iw = LG_IX(c.G, ji, jk, l + 1);
+    g.ro_b = ro[iw];
+    g.vcw = VF == VF_LIQUID ? c.w.vfall_cw[iw] : 0.0;
+    return g;
+  }
+  __device__ __forceinline__ GenIn inputs(const In &g, int l) const {
+    const double *p = stage + (l - 1) % (2 * KX) * NS * BCOL;
+    GenIn i;
+    i.tr = (double)g.tr;
+    i.ro_b = g.ro_b;
+    i.vcw = g.vcw;
+    i.wo = p[GS_WO * BCOL];
+    i.wn = p[GS_WN * BCOL];
+    i.az = p[GS_AZ * BCOL];
+    i.Vb = p[GS_V * BCOL];
+    i.qb = p[GS_QB * BCOL];
+    i.tif = 0.0;
+    i.ct = HEAT && COND ? p[(CP == CP_ICE ? GS_CI : GS_CW) * BCOL] : 0.0;
+    return i;
+  }
+  // Thomas elimination of the row of layer l
+  __device__ __forceinline__ void eliminate(int l) {
+    const double den = row.d - ep * cprev;
+    const double epq = row.e / den;
+    const double rpq = (row.r - rp * cprev) / den;
+    if (OWN_EP) ep_col[(l - 1) * BCOL] = epq;
+    ep = epq;
+    rp = rpq;
+    cprev = row.cq;
+  }
+  // builds the row of layer l and eliminates the one above it, whose r' becomes element (l-1) % GR_PART of part P
+  template <int P, int U>
+  __device__ __forceinline__ void step(int l) {
+    const GenIn cur = inputs(in[U], l);
+    GenRow nxt;
+    if (P == 0 && U == 0 && l == 1) {
+      nxt = gen_row<VF, CP, HEAT, POS_TOP>(cur, s, vf_const, dt, V, az_sfc, t_sfc, hb_on, l, nl);
+    } else if (l < nl) {
+      nxt = gen_row<VF, CP, HEAT, POS_MID>(cur, s, vf_const, dt, V, az_sfc, t_sfc, hb_on, l, nl);
+      eliminate(l - 1);
+      r[P][l - 1 - P * GR_PART] = rp;
+    } else {
+      nxt = gen_row<VF, CP, HEAT, POS_BOTTOM>(cur, s, vf_const, dt, V, az_sfc, t_sfc, hb_on, l, nl);
+      eliminate(l - 1);
+      r[P][l - 1 - P * GR_PART] = rp;
+      if (HEAT && COND) hb[t * BCOL] = nxt.hb;
+    }
+    V = cur.Vb;
+    if (HEAT && COND) ha[((l - 1) % (2 * KX) * NCS + t) * BCOL] = nxt.ha;
+    in[U] = load(l + 4 <= nl ? l + 4 : nl);
+    row = nxt;
+  }
+  template <int P>
+  __device__ __forceinline__ void sweep() {
+    if constexpr (P < GR_PARTS) {
+      if (P * GR_PART >= nl) return;
+      const int to = nl < (P + 1) * GR_PART ? nl : (P + 1) * GR_PART;
+      for (int l = P * GR_PART + 1; l <= to; l += 4) {
+        __syncthreads();
+        step<P, 0>(l);
+        if (l + 1 <= to) step<P, 1>(l + 1);
+        if (KX == 2 && l + 2 <= to) __syncthreads();
+        if (l + 2 <= to) step<P, 2>(l + 2);
+        if (l + 3 <= to) step<P, 3>(l + 3);
+      }
+      sweep<P + 1>();
+    }
+  }
+  __device__ __forceinline__ void forward() {
+    const ix_t i1 = LG_IX(c.G, ji, jk, 1);
+    s.fi_up = s.fr_up = s.fe_up = 0.0;
+    s.ro_cur = ro[i1];
+    V = c.g64.volume[i1];
+    s.q = 0.5 * dt / V;
+    s.vcw_lo = VF == VF_LIQUID ? c.w.vfall_cw[i1] : 0.0;
+    ep = rp = cprev = 0.0;
+    row = GenRow{};
+#pragma unroll
+    for (int u = 0; u < 4; ++u) in[u] = load(1 + u <= nl ? 1 + u : nl);
+    sweep<0>();
+    eliminate(nl);
+    __syncthreads();  // the last heating terms, rain's e'
+  }
+  // back substitution and clipping of round-off negatives (gen_back); x: the level below
+  template <int P>
+  __device__ __forceinline__ void back(Fld<double> rn, bool active, double &x, bool &finite) {
+    if constexpr (P >= 0) {
+      if (P * GR_PART < nl) {
+        const int top = nl < (P + 1) * GR_PART ? nl : (P + 1) * GR_PART;
+#pragma unroll 4
+        for (int l = top; l > P * GR_PART && l > 1; --l) {  // from x(l) to x(l-1)
+          x = r[P][l - 1 - P * GR_PART] - ep_col[(l - 2) * BCOL] * x;
+          if (active) rn[LG_IX(c.G, ji, jk, l - 1)] = x < 0.0 ? 0.0 : x;
+          finite = finite && isfinite(x);
+        }
+      }
+      back<P - 1>(rn, active, x, finite);
+    }
+  }
+  __device__ __forceinline__ void backward(Fld<double> rn, bool active) {
+    double x = rp;
+    if (active) rn[LG_IX(c.G, ji, jk, nl)] = x < 0.0 ? 0.0 : x;
+    bool finite = isfinite(x);
+    back<GR_PARTS - 1>(rn, active, x, finite);
+    if (!HEAT && !finite && active) atomicOr(c.C.nonfinite, 1ull);  // the corrector's new values
+  }
+};
+
+template <class R, bool HEAT>
+struct GenStager {
+  static constexpr int KX = gr_k(HEAT), NS = gr_fields(HEAT);
+  struct In {
+    double wo, wn, az, V;
+    R tif;
+  };
+  const CtxT<R> &c;
+  const StateDev &old, &nw;
+  double *stage;
+  const double *ha, *hb;
+  const int ji, jk, nl;
+  const bool active;
+  const double dt;
+  In in[4];
+  __device__ __forceinline__ In load(int l) const {
+    const ix_t iw = LG_IX(c.G, ji, jk, l + 1);
+    In g;
+    g.wo = old.wind_w[iw];
+    g.wn = nw.wind_w[iw];
+    g.az = c.g64.area_z[iw];
+    g.V = c.g64.volume[iw];
+    g.tif = HEAT ? c.w.temperature[iw] : R(0.0);
+    return g;
+  }
+  // leaves level l in the ring; past the bottom its slots are not read any more
+  template <int U>
+  __device__ __forceinline__ void put(int l) {
+    double *p = stage + (l - 1) % (2 * KX) * NS * BCOL;
+    const In g = in[U];
+    p[GS_WO * BCOL] = g.wo;
+    p[GS_WN * BCOL] = g.wn;
+    p[GS_AZ * BCOL] = g.az;
+    p[GS_V * BCOL] = g.V;
+    p[GS_QB * BCOL] = 0.5 * dt / g.V;
+    if (HEAT) {
+      const double tif = (double)g.tif;
+      p[GS_CI * BCOL] = c_p_ice(tif) * tif;
+      p[GS_CW * BCOL] = c_p_water_sel(tif) * tif;
+    }
+    in[U] = load(l + 4 <= nl ? l + 4 : nl);
+  }
+  // adds up the heating of the layers from..from+KX-1 in constituent order
+  __device__ __forceinline__ void heat(int from) {
+    if (!HEAT || !active) return;
+    for (int l = from; l < from + KX && l <= nl; ++l) {
+      double csh = 0.0;
+#pragma unroll
+      for (int q = 0; q < NCS; ++q) {
+        csh = csh + ha[((l - 1) % (2 * KX) * NCS + q) * BCOL];
+        if (l == nl) csh = csh - hb[q * BCOL];
+      }
+      c.w.csh[LG_IX(c.G, ji, jk, l)] = (R)csh;
+    }
+  }
+  __device__ __forceinline__ void run() {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) in[u] = load(1 + u <= nl ? 1 + u : nl);
+    put<0>(1);
+    put<1>(2);
+    if (KX == 4) put<2>(3), put<3>(4);
+    for (int l = 1; l <= nl; l += 4) {
+      __syncthreads();  // the tracers start with level l
+      if (KX == 4) {
+        put<0>(l + 4);
+        put<1>(l + 5);
+        put<2>(l + 6);
+        put<3>(l + 7);
+      } else {
+        put<2>(l + 2);
+        put<3>(l + 3);
+        if (l > 1) heat(l - 2);
+        if (l + 2 <= nl) {
+          __syncthreads();  // ... with level l+2
+          put<0>(l + 4);
+          put<1>(l + 5);
+          heat(l);
+        }
+      }
+    }
+    __syncthreads();
+    heat((nl - 1) / KX * KX + 1);
+  }
+};
+
+template <class R, int VF, int CP, bool HEAT, bool OWN_EP = true>
+__device__ __forceinline__ void gen_tracer(const CtxT<R> &c, const StateDev &old, const StateDev &nw, double *lds, int t, int lane,
+                                           bool active, int ji, int jk, int jc, double vf_const) {
+  const int nl = c.G.nl;
+  double *stage = lds + (size_t)GR_EP * nl * BCOL, *ha = stage + 2 * gr_k(HEAT) * gr_fields(HEAT) * BCOL,
+         *hb = ha + 2 * gr_k(HEAT) * NCS * BCOL;
+  GenTracer<R, VF, CP, HEAT, OWN_EP> g{c,
+                                       stage + lane,
+                                       ha + lane,
+                                       hb + lane,
+                                       lds + (OWN_EP ? t : 1) * nl * BCOL + lane,  // (without its own: rain's)
+                                       old.rho[jc - 1],
+                                       c.w.tend_rho[jc - 1],
+                                       t,
+                                       ji,
+                                       jk,
+                                       nl,
+                                       c.C.dtime,
+                                       vf_const,
+                                       AT(c.g64.area_z, ji, jk, nl + 1),
+                                       HEAT && CP != CP_NONE ? (double)AT(c.w.temperature, ji, jk, nl) : 0.0,
+                                       jc > c.G.ncond / 4};
+  g.forward();
+  g.backward(nw.rho[jc - 1], active);
+}
+template <class R, bool HEAT>
+__device__ __forceinline__ void b_gen_reg(const CtxT<R> &c, const StateDev &old, const StateDev &nw, const Bid bid, double *lds) {
+  const int nx = c.G.nx, nl = c.G.nl;
+  const int lane = threadIdx.x, t = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const int wpr = col_waves_per_row(nx);
+  const int ji = bid.x / wpr + 1, jk_raw = (bid.x % wpr) * BCOL + lane + 1;
+  const bool active = jk_raw <= nx;
+  const int jk = active ? jk_raw : nx;  // idle lanes mirror a valid column, store nothing
+  const double vf_snow = v_fall_solid(500.e-6), vf_ice = v_fall_solid(95.e-6);
+  switch (t) {  // the kinds of gen_dispatch
+    case 0: gen_tracer<R, VF_CONST, CP_ICE, HEAT>(c, old, nw, lds, t, lane, active, ji, jk, 1, vf_snow); break;
+    case 1: gen_tracer<R, VF_NONE, HEAT ? CP_WATER : CP_NONE, HEAT>(c, old, nw, lds, t, lane, active, ji, jk, 2, 0.0); break;
+    case 2: gen_tracer<R, VF_CONST, CP_ICE, HEAT>(c, old, nw, lds, t, lane, active, ji, jk, 3, vf_ice); break;
+    case 3: gen_tracer<R, VF_LIQUID, CP_WATER, HEAT>(c, old, nw, lds, t, lane, active, ji, jk, 4, 0.0); break;
+    case 4: gen_tracer<R, VF_NONE, HEAT ? CP_ICE : CP_NONE, HEAT, false>(c, old, nw, lds, t, lane, active, ji, jk, 5, 0.0); break;
+    case 5: gen_tracer<R, VF_NONE, CP_NONE, HEAT, false>(c, old, nw, lds, t, lane, active, ji, jk, 7, 0.0); break;
+    default: {
+      double *stage = lds + (size_t)GR_EP * nl * BCOL, *ha = stage + 2 * gr_k(HEAT) * gr_fields(HEAT) * BCOL;
+      GenStager<R, HEAT> g{c, old, nw, stage + lane, ha + lane, ha + 2 * gr_k(HEAT) * NCS * BCOL + lane, ji, jk, nl, active, c.C.dtime};
+      g.run();
+    }
+  }
+}
+template <class R, bool HEAT>
+__global__ void __launch_bounds__(BCOL *GR_WAVES) k_gen_reg(const CtxT<R> c, const StateDev old, const StateDev nw) {
+  extern __shared__ double lds[];
+  b_gen_reg<R, HEAT>(c, old, nw, bid_here(), lds);
+}
+template <class R>
+void launch_solve_gen(const CtxT<R> &c, const StateDev &old, const StateDev &nw, int rk, hipStream_t st) {
+  const int waves = col_waves(c.G);
+  if (gen_reg(c.G.nl)) {
+    const dim3 g((unsigned)waves), b(BCOL, GR_WAVES);
+    const size_t l = gr_lds_bytes(c.G.nl, rk == 1);
+    if (rk == 1)
+      hipLaunchKernelGGL((k_gen_reg<R, true>), g, b, l, st, c, old, nw);
+    else
+      hipLaunchKernelGGL((k_gen_reg<R, false>), g, b, l, st, c, old, nw);
+    return;
+  }
+  hipLaunchKernelGGL(k_solve_gen<R>, dim3((unsigned)((waves + GEN_GROUPS - 1) / GEN_GROUPS)), dim3(BCOL, NTR * GEN_GROUPS), 0, st, c, old,
+                     nw, rk);
+}
+template void launch_solve_gen<double>(const CtxT<double> &, const StateDev &, const StateDev &, int, hipStream_t);
+template void launch_solve_gen<float>(const CtxT<float> &, const StateDev &, const StateDev &, int, hipStream_t);
+
 template __global__ void k_solve_ver<double>(const CtxT<double>, const StateDev, const StateDev, int);
 template __global__ void k_solve_ver<float>(const CtxT<float>, const StateDev, const StateDev, int);
-template __global__ void k_solve_gen<double>(const CtxT<double>, const StateDev, const StateDev, int);
-template __global__ void k_solve_gen<float>(const CtxT<float>, const StateDev, const StateDev, int);
 
 // ---- the same kernels over a group of domains (one launch per phase) ------------------------
 LG_BATCH_KERNEL(solve_ver, BCOL, PH_SOLVE_VER, b_solve_ver(d.c, d.s[a.old_slot], d.s[a.new_slot], a.rk, bid))
@@ -1115,6 +1424,14 @@ __global__ void __launch_bounds__(VS_THREADS, 2)
   b_ver_seg<R, RK, K>(d.c, d.s[a.old_slot], d.s[a.new_slot], bid, lds);
 }
 LG_BATCH_KERNEL(solve_gen, BCOL * NTR * GEN_GROUPS, PH_SOLVE_GEN, b_solve_gen(d.c, d.s[a.old_slot], d.s[a.new_slot], a.rk, bid))
+template <class R, bool HEAT>
+__global__ void __launch_bounds__(BCOL *GR_WAVES)
+    kb_gen_reg(const MemberDev<R> *__restrict__ M, const int *__restrict__ prefix, int nm, const BatchArgs a) {
+  extern __shared__ double lds[];
+  Bid bid;
+  const MemberDev<R> &d = batch_block(M, prefix, nm, PH_GEN_REG, bid);
+  b_gen_reg<R, HEAT>(d.c, d.s[a.old_slot], d.s[a.new_slot], bid, lds);
+}
 
 template <class R>
 bool batch_launch_solve(int ph, dim3 g, dim3 b, hipStream_t st, const MemberDev<R> *M, const int *prefix, int nm, const BatchArgs &a) {
@@ -1130,6 +1447,14 @@ bool batch_launch_solve(int ph, dim3 g, dim3 b, hipStream_t st, const MemberDev<
   } while (0)
     LG_VS_DISPATCH(a.nl_max);
 #undef LG_VS
+    return true;
+  }
+  if (ph == PH_GEN_REG) {
+    const size_t l = gr_lds_bytes(a.nl_max < GR_MAX_NL ? a.nl_max : GR_MAX_NL, a.rk == 1);
+    if (a.rk == 1)
+      hipLaunchKernelGGL((kb_gen_reg<R, true>), g, b, l, st, M, prefix, nm, a);
+    else
+      hipLaunchKernelGGL((kb_gen_reg<R, false>), g, b, l, st, M, prefix, nm, a);
     return true;
   }
   if (ph == PH_SOLVE_GEN) {

@@ -19,7 +19,6 @@ template <class R> __global__ void k_pgrad_vt(const CtxT<R> c, const StateDev ol
 // the second substep's vorticity flux term (and kinetic-energy gradient) with its wind update
 template <class R> __global__ void k_vort_flux_vt(const CtxT<R> c, const StateDev old, const StateDev nw, int with_ke_grad);
 template <class R> __global__ void k_solve_ver(const CtxT<R> c, const StateDev old, const StateDev nw, int rk);
-template <class R> __global__ void k_solve_gen(const CtxT<R> c, const StateDev old, const StateDev nw, int rk);
 template <class R> __global__ void k_diff_zeta(const CtxT<R> c, const StateDev s);
 template <class R> __global__ void k_diff_coef(const CtxT<R> c, const StateDev s);
 template <class R> __global__ void k_diff_coef2(const CtxT<R> c, const StateDev s);  // nx even: two cells per thread
@@ -106,6 +105,20 @@ __host__ __device__ inline int col_waves(const Geom &G) { return col_waves_per_r
 // block of six would land 2,2,1,1 and leave room for only one block per CU.
 constexpr int NTR = 6;         // tracers per moist column
 constexpr int GEN_GROUPS = 2;  // 64-column groups per block
+// The tracer solver with the eliminated coefficients in registers and LDS (k_gen_reg): r' of GR_PARTS x GR_PART
+// levels per lane, e' of the GR_EP tracers that have their own, a ring of 2 x gr_k levels of gr_fields values
+// that the tracers share and of heating terms; a wavefront per tracer and one that fills the ring
+constexpr int GR_PART = 16, GR_PARTS = 4, GR_EP = 4, GR_WAVES = NTR + 1;
+__host__ __device__ constexpr int gr_k(bool heat) { return heat ? 2 : 4; }
+__host__ __device__ constexpr int gr_fields(bool heat) { return heat ? 7 : 5; }
+__host__ __device__ inline size_t gr_lds_bytes(int nl, bool heat) {
+  return sizeof(double) * 64 * ((size_t)GR_EP * nl + 2 * gr_k(heat) * gr_fields(heat) + (heat ? 2 * gr_k(heat) * 5 + 5 : 0));
+}
+// Columns that fit take it whatever the domain's size; taller ones go through the column scratch (k_solve_gen).
+constexpr int GR_MAX_NL = GR_PART * GR_PARTS;
+__host__ __device__ inline bool gen_reg(int nl) { return nl <= GR_MAX_NL; }
+template <class R>
+void launch_solve_gen(const CtxT<R> &c, const StateDev &old, const StateDev &nw, int rk, hipStream_t st);
 
 // Levels 1..diss_levels in which k_dissipation forms the dissipation rate: with a friction of the wind
 // all of them, with the Klemp layer alone those whose upper or lower interface lies in it (below it

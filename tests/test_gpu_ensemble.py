@@ -177,6 +177,41 @@ def test_third_order_theta_columns_match_oracle(ny, nx, nl, oro, moist, rows, se
     assert all(np.array_equal(got[k], want[k]) for k in want)
 
 
+@pytest.mark.parametrize("nl,nx", [(3, 5), (4, 63), (5, 64), (16, 65), (17, 7), (18, 7), (31, 128), (33, 129), (48, 9), (50, 9), (63, 64),
+                                   (64, 70)])
+def test_tracer_solver_levels_match_oracle(nl, nx):
+    """The tracer solver keeps up to 64 levels in parts of 16, filled and emptied in chunks of 2 and 4: the
+    smallest columns, the ends of chunks and parts, the tallest column that fits, bitwise against the oracle."""
+    cfg = dataclasses.replace(tiny_config(ny=3, nx=nx, n_layers=nl, moist=True), n_oro_layers=max(1, nl - 4))
+    g, st = make_case(cfg, cloud_frac=0.3)
+    want = _oracle(cfg, g, st, 3)
+    s = Step(cfg, g)
+    s.start(st)
+    s.run(0, 3)
+    got = s.get_state(1)
+    s.close()
+    assert all(np.array_equal(got[k], want[k]) for k in want)
+
+
+def test_batched_tracer_solver_with_members_of_different_height():
+    cfgs = [tiny_config(ny=4 + i, nx=30 + 40 * i, n_layers=nl, moist=True) for i, nl in enumerate((66, 7, 64, 70))]
+    cases = [make_case(c, cloud_frac=0.3) for c in cfgs]
+    steps = []
+    for c, (g, st) in zip(cfgs, cases):
+        s = Step(c, g)
+        s.start(st)
+        steps.append(s)
+    e = Ensemble(steps)
+    e.run(0, 3, mode=Ensemble.BATCHED)
+    e.sync()
+    for c, (g, st), s in zip(cfgs, cases, steps):
+        got, want = s.get_state(1), _oracle(c, g, st, 3)
+        assert all(np.array_equal(got[k], want[k]) for k in want), c.n_layers
+    e.close()
+    for s in steps:
+        s.close()
+
+
 def test_vertical_solver_default_passes_by_size():
     """One pass per column once the domain has as many 64-column wavefronts as the GPU has SIMDs."""
     for n, want in ((128, 3), (256, 1)):
