@@ -18,13 +18,13 @@ namespace lgame {
 // PH_PGRAD is the first substep's pressure gradient with its wind update (b_pgrad_vt), PH_VORT_FLUX_VT
 // the second substep's vorticity flux term with its wind update (b_vort_flux_vt); PH_VEC_TEND is the
 // second substep's wind update alone (runs without momentum advection).  PH_VER_SEG takes the place of
-// PH_SOLVE_VER when ver_segments holds for every member.  PH_GEN_REG runs the members for which gen_reg
-// holds, PH_SOLVE_GEN the others.
+// PH_SOLVE_VER when ver_segments holds for every member.  PH_GEN_REG and PH_GEN_TALL run the members
+// for which gen_reg holds (the latter those of gr_tall), PH_SOLVE_GEN the others.
 enum Phase : int {
   PH_TEMPERATURE, PH_SFC_TURB, PH_THETA_DIV, PH_THETA_EDGE, PH_PGRAD, PH_POT_VORT,
   PH_VORT_FLUX, PH_DIFF_ZETA, PH_DIFF_COEF, PH_DIFF_DUAL, PH_DIFF_MOM, PH_PBL_WIND,
   PH_DISSIPATION, PH_VEC_TEND, PH_DIFF_FLUX, PH_SCALAR, PH_SURFACE, PH_SOLVE_VER, PH_SOLVE_GEN, PH_RAD,
-  PH_VORT_FLUX_VT, PH_VER_SEG, PH_GEN_REG,
+  PH_VORT_FLUX_VT, PH_VER_SEG, PH_GEN_REG, PH_GEN_TALL,
   PH_COUNT
 };
 
@@ -88,8 +88,9 @@ __host__ __device__ inline void phase_grid(int ph, const Geom &G, int by, int se
     case PH_SOLVE_VER: gx = col_waves(G); gy = gz = 1; return;
     case PH_VER_SEG: gx = vs_blocks_per_row(G.nx) * G.ny; gy = gz = 1; return;
     case PH_RAD: gx = (nx * ny + BCOL - 1) / BCOL; gy = gz = 1; return;
-    // (each member in one of the two, the other has no blocks of it)
-    case PH_GEN_REG: gx = gen_reg(G.nl) ? col_waves(G) : 0; gy = gz = 1; return;
+    // (each member in one of the three, the others have no blocks of it)
+    case PH_GEN_REG: gx = gr_tall(G.nl) ? 0 : col_waves(G); gy = gz = 1; return;
+    case PH_GEN_TALL: gx = gr_tall(G.nl) && gen_reg(G.nl) ? col_waves(G) : 0; gy = gz = 1; return;
     case PH_SOLVE_GEN: gx = gen_reg(G.nl) ? 0 : (col_waves(G) + GEN_GROUPS - 1) / GEN_GROUPS; gy = gz = 1; return;
     default: return;
   }

@@ -1764,7 +1764,7 @@ int enqueue_group(lgame_ensemble *e, BatchGroup &g, int a_slot, int b_slot, int 
       blk = dim3(BCOL);
     else if (ph == PH_VER_SEG)
       blk = dim3(VS_THREADS);
-    else if (ph == PH_GEN_REG)
+    else if (ph == PH_GEN_REG || ph == PH_GEN_TALL)
       blk = dim3(BCOL, GR_WAVES);
     else if (ph == PH_SOLVE_GEN)
       blk = dim3(BCOL, NTR * GEN_GROUPS);
@@ -1847,8 +1847,9 @@ int enqueue_group(lgame_ensemble *e, BatchGroup &g, int a_slot, int b_slot, int 
     launch(PH_SCALAR, a);
     if (C.lsoil || C.lsens) launch(PH_SURFACE, a);
     launch(ver_segments(g.nl_max) ? PH_VER_SEG : PH_SOLVE_VER, a);
-    if (g.moist && g.total[PH_GEN_REG]) launch(PH_GEN_REG, a);
-    if (g.moist && g.total[PH_SOLVE_GEN]) launch(PH_SOLVE_GEN, a);
+    if (g.moist)
+      for (int ph : {PH_GEN_REG, PH_GEN_TALL, PH_SOLVE_GEN})
+        if (g.total[ph]) launch(ph, a);
   }
   ECHK(e, hipGetLastError());
   return 0;

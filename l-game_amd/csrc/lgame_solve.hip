@@ -1112,19 +1112,21 @@ __global__ void __launch_bounds__(BCOL * NTR * GEN_GROUPS) k_solve_gen(const Ctx
 // up the sediment heating.  The tracer wavefronts load only their density and tendency, four levels ahead.
 // One barrier per KX levels: behind it the tracers read levels of the ring while the next KX are written,
 // and leave heating terms while those of the previous KX are added up.  KX is 4, or 2 with the heating, where
-// the ring holds more.
+// the ring holds more; half of that in columns of 65 to 72 layers (TALL), whose e' leaves less LDS.
 // Bound by memory traffic (the scratch was 160 of 350 B per tracer column and level): us per launch at the
 // predictor and the corrector, k_solve_gen -> here: 512x512x60 FP64 1240, 1030 -> 880, 718 (4.5 TB/s), mixed
-// 1190, 990 -> 851, 703; 257x193x55 FP64 240 -> 203, 162.  Without the seventh wavefront (each tracer loading
-// everything, two levels ahead) it was bound by latency: 1517, 991.
+// 1190, 990 -> 851, 703; 257x193x55 FP64 240 (mean) -> 203, 162; tall, 291x209x69 mixed 428 (mean) -> 352, 255.
+// Without the seventh wavefront (each tracer loading everything, two levels ahead) it was bound by latency:
+// 1517, 991.
 typedef double GenVec __attribute__((ext_vector_type(GR_PART)));
+typedef double GenVecLast __attribute__((ext_vector_type(GR_LAST)));  // the last part of a tall column
 enum { GS_WO, GS_WN, GS_AZ, GS_V, GS_QB, GS_CI, GS_CW };  // what the ring holds of a level: ... c_p T of ice, of water
 
 // One tracer.  stage: the ring, ep_col: e' of level 1 (levels BCOL apart), all at this lane
-template <class R, int VF, int CP, bool HEAT, bool OWN_EP>
+template <class R, int VF, int CP, bool HEAT, bool TALL, bool OWN_EP>
 struct GenTracer {
   static constexpr bool COND = CP != CP_NONE;
-  static constexpr int KX = gr_k(HEAT), NS = gr_fields(HEAT);
+  static constexpr int KX = gr_k(HEAT, TALL), NS = gr_fields(HEAT);
   struct In {
     R tr;  // converted where it is used, so that nothing waits for the load here
     double ro_b, vcw;
@@ -1141,6 +1143,7 @@ struct GenTracer {
   GenRow row;
   double V, ep, rp, cprev;
   GenVec r[GR_PARTS];
+  GenVecLast r_last;
   In in[4];
 
   __device__ __forceinline__ In load(int l) const {
@@ -1176,7 +1179,22 @@ struct GenTracer {
     rp = rpq;
     cprev = row.cq;
   }
-  // builds the row of layer l and eliminates the one above it, whose r' becomes element (l-1) % GR_PART of part P
+  // r' of layer l-1: element (l-1) % GR_PART of part P
+  template <int P>
+  __device__ __forceinline__ void keep(int l) {
+    if constexpr (P < GR_PARTS)
+      r[P][l - 1 - P * GR_PART] = rp;
+    else
+      r_last[l - 1 - P * GR_PART] = rp;
+  }
+  template <int P>
+  __device__ __forceinline__ double kept(int l) const {
+    if constexpr (P < GR_PARTS)
+      return r[P][l - 1 - P * GR_PART];
+    else
+      return r_last[l - 1 - P * GR_PART];
+  }
+  // builds the row of layer l and eliminates the one above it
   template <int P, int U>
   __device__ __forceinline__ void step(int l) {
     const GenIn cur = inputs(in[U], l);
@@ -1186,11 +1204,11 @@ struct GenTracer {
     } else if (l < nl) {
       nxt = gen_row<VF, CP, HEAT, POS_MID>(cur, s, vf_const, dt, V, az_sfc, t_sfc, hb_on, l, nl);
       eliminate(l - 1);
-      r[P][l - 1 - P * GR_PART] = rp;
+      keep<P>(l);
     } else {
       nxt = gen_row<VF, CP, HEAT, POS_BOTTOM>(cur, s, vf_const, dt, V, az_sfc, t_sfc, hb_on, l, nl);
       eliminate(l - 1);
-      r[P][l - 1 - P * GR_PART] = rp;
+      keep<P>(l);
       if (HEAT && COND) hb[t * BCOL] = nxt.hb;
     }
     V = cur.Vb;
@@ -1200,15 +1218,17 @@ struct GenTracer {
   }
   template <int P>
   __device__ __forceinline__ void sweep() {
-    if constexpr (P < GR_PARTS) {
+    if constexpr (P < (TALL ? GR_PARTS + 1 : GR_PARTS)) {
       if (P * GR_PART >= nl) return;
       const int to = nl < (P + 1) * GR_PART ? nl : (P + 1) * GR_PART;
       for (int l = P * GR_PART + 1; l <= to; l += 4) {
         __syncthreads();
         step<P, 0>(l);
+        if (KX == 1 && l + 1 <= to) __syncthreads();
         if (l + 1 <= to) step<P, 1>(l + 1);
-        if (KX == 2 && l + 2 <= to) __syncthreads();
+        if (KX <= 2 && l + 2 <= to) __syncthreads();
         if (l + 2 <= to) step<P, 2>(l + 2);
+        if (KX == 1 && l + 3 <= to) __syncthreads();
         if (l + 3 <= to) step<P, 3>(l + 3);
       }
       sweep<P + 1>();
@@ -1237,7 +1257,7 @@ struct GenTracer {
         const int top = nl < (P + 1) * GR_PART ? nl : (P + 1) * GR_PART;
 #pragma unroll 4
         for (int l = top; l > P * GR_PART && l > 1; --l) {  // from x(l) to x(l-1)
-          x = r[P][l - 1 - P * GR_PART] - ep_col[(l - 2) * BCOL] * x;
+          x = kept<P>(l) - ep_col[(l - 2) * BCOL] * x;
           if (active) rn[LG_IX(c.G, ji, jk, l - 1)] = x < 0.0 ? 0.0 : x;
           finite = finite && isfinite(x);
         }
@@ -1249,14 +1269,14 @@ struct GenTracer {
     double x = rp;
     if (active) rn[LG_IX(c.G, ji, jk, nl)] = x < 0.0 ? 0.0 : x;
     bool finite = isfinite(x);
-    back<GR_PARTS - 1>(rn, active, x, finite);
+    back<TALL ? GR_PARTS : GR_PARTS - 1>(rn, active, x, finite);
     if (!HEAT && !finite && active) atomicOr(c.C.nonfinite, 1ull);  // the corrector's new values
   }
 };
 
-template <class R, bool HEAT>
+template <class R, bool HEAT, bool TALL>
 struct GenStager {
-  static constexpr int KX = gr_k(HEAT), NS = gr_fields(HEAT);
+  static constexpr int KX = gr_k(HEAT, TALL), NS = gr_fields(HEAT);
   struct In {
     double wo, wn, az, V;
     R tif;
@@ -1309,43 +1329,43 @@ struct GenStager {
       c.w.csh[LG_IX(c.G, ji, jk, l)] = (R)csh;
     }
   }
+  // the KX levels from l on, whose first is input U
+  template <int U, int K>
+  __device__ __forceinline__ void puts(int l) {
+    if constexpr (K < KX) {
+      put<(U + K) % 4>(l + K);
+      puts<U, K + 1>(l);
+    }
+  }
+  // while the tracers work on the KX levels from l on (input U): the next levels, the heating of the previous ones
+  template <int U>
+  __device__ __forceinline__ void chunk(int l) {
+    if (U > 0 && l > nl) return;
+    __syncthreads();
+    puts<U + KX, 0>(l + KX);
+    if (l > 1) heat(l - KX);
+  }
   __device__ __forceinline__ void run() {
 #pragma unroll
     for (int u = 0; u < 4; ++u) in[u] = load(1 + u <= nl ? 1 + u : nl);
-    put<0>(1);
-    put<1>(2);
-    if (KX == 4) put<2>(3), put<3>(4);
+    puts<0, 0>(1);
     for (int l = 1; l <= nl; l += 4) {
-      __syncthreads();  // the tracers start with level l
-      if (KX == 4) {
-        put<0>(l + 4);
-        put<1>(l + 5);
-        put<2>(l + 6);
-        put<3>(l + 7);
-      } else {
-        put<2>(l + 2);
-        put<3>(l + 3);
-        if (l > 1) heat(l - 2);
-        if (l + 2 <= nl) {
-          __syncthreads();  // ... with level l+2
-          put<0>(l + 4);
-          put<1>(l + 5);
-          heat(l);
-        }
-      }
+      chunk<0>(l);
+      if (KX < 4) chunk<KX % 4>(l + KX);
+      if (KX < 2) chunk<2>(l + 2), chunk<3>(l + 3);
     }
     __syncthreads();
     heat((nl - 1) / KX * KX + 1);
   }
 };
 
-template <class R, int VF, int CP, bool HEAT, bool OWN_EP = true>
+template <class R, int VF, int CP, bool HEAT, bool TALL, bool OWN_EP = true>
 __device__ __forceinline__ void gen_tracer(const CtxT<R> &c, const StateDev &old, const StateDev &nw, double *lds, int t, int lane,
                                            bool active, int ji, int jk, int jc, double vf_const) {
   const int nl = c.G.nl;
-  double *stage = lds + (size_t)GR_EP * nl * BCOL, *ha = stage + 2 * gr_k(HEAT) * gr_fields(HEAT) * BCOL,
-         *hb = ha + 2 * gr_k(HEAT) * NCS * BCOL;
-  GenTracer<R, VF, CP, HEAT, OWN_EP> g{c,
+  double *stage = lds + (size_t)GR_EP * nl * BCOL, *ha = stage + 2 * gr_k(HEAT, TALL) * gr_fields(HEAT) * BCOL,
+         *hb = ha + 2 * gr_k(HEAT, TALL) * NCS * BCOL;
+  GenTracer<R, VF, CP, HEAT, TALL, OWN_EP> g{c,
                                        stage + lane,
                                        ha + lane,
                                        hb + lane,
@@ -1364,7 +1384,7 @@ __device__ __forceinline__ void gen_tracer(const CtxT<R> &c, const StateDev &old
   g.forward();
   g.backward(nw.rho[jc - 1], active);
 }
-template <class R, bool HEAT>
+template <class R, bool HEAT, bool TALL>
 __device__ __forceinline__ void b_gen_reg(const CtxT<R> &c, const StateDev &old, const StateDev &nw, const Bid bid, double *lds) {
   const int nx = c.G.nx, nl = c.G.nl;
   const int lane = threadIdx.x, t = __builtin_amdgcn_readfirstlane(threadIdx.y);
@@ -1374,34 +1394,40 @@ __device__ __forceinline__ void b_gen_reg(const CtxT<R> &c, const StateDev &old,
   const int jk = active ? jk_raw : nx;  // idle lanes mirror a valid column, store nothing
   const double vf_snow = v_fall_solid(500.e-6), vf_ice = v_fall_solid(95.e-6);
   switch (t) {  // the kinds of gen_dispatch
-    case 0: gen_tracer<R, VF_CONST, CP_ICE, HEAT>(c, old, nw, lds, t, lane, active, ji, jk, 1, vf_snow); break;
-    case 1: gen_tracer<R, VF_NONE, HEAT ? CP_WATER : CP_NONE, HEAT>(c, old, nw, lds, t, lane, active, ji, jk, 2, 0.0); break;
-    case 2: gen_tracer<R, VF_CONST, CP_ICE, HEAT>(c, old, nw, lds, t, lane, active, ji, jk, 3, vf_ice); break;
-    case 3: gen_tracer<R, VF_LIQUID, CP_WATER, HEAT>(c, old, nw, lds, t, lane, active, ji, jk, 4, 0.0); break;
-    case 4: gen_tracer<R, VF_NONE, HEAT ? CP_ICE : CP_NONE, HEAT, false>(c, old, nw, lds, t, lane, active, ji, jk, 5, 0.0); break;
-    case 5: gen_tracer<R, VF_NONE, CP_NONE, HEAT, false>(c, old, nw, lds, t, lane, active, ji, jk, 7, 0.0); break;
+    case 0: gen_tracer<R, VF_CONST, CP_ICE, HEAT, TALL>(c, old, nw, lds, t, lane, active, ji, jk, 1, vf_snow); break;
+    case 1: gen_tracer<R, VF_NONE, HEAT ? CP_WATER : CP_NONE, HEAT, TALL>(c, old, nw, lds, t, lane, active, ji, jk, 2, 0.0); break;
+    case 2: gen_tracer<R, VF_CONST, CP_ICE, HEAT, TALL>(c, old, nw, lds, t, lane, active, ji, jk, 3, vf_ice); break;
+    case 3: gen_tracer<R, VF_LIQUID, CP_WATER, HEAT, TALL>(c, old, nw, lds, t, lane, active, ji, jk, 4, 0.0); break;
+    case 4: gen_tracer<R, VF_NONE, HEAT ? CP_ICE : CP_NONE, HEAT, TALL, false>(c, old, nw, lds, t, lane, active, ji, jk, 5, 0.0); break;
+    case 5: gen_tracer<R, VF_NONE, CP_NONE, HEAT, TALL, false>(c, old, nw, lds, t, lane, active, ji, jk, 7, 0.0); break;
     default: {
-      double *stage = lds + (size_t)GR_EP * nl * BCOL, *ha = stage + 2 * gr_k(HEAT) * gr_fields(HEAT) * BCOL;
-      GenStager<R, HEAT> g{c, old, nw, stage + lane, ha + lane, ha + 2 * gr_k(HEAT) * NCS * BCOL + lane, ji, jk, nl, active, c.C.dtime};
+      double *stage = lds + (size_t)GR_EP * nl * BCOL, *ha = stage + 2 * gr_k(HEAT, TALL) * gr_fields(HEAT) * BCOL;
+      GenStager<R, HEAT, TALL> g{c, old, nw, stage + lane, ha + lane, ha + 2 * gr_k(HEAT, TALL) * NCS * BCOL + lane, ji, jk, nl, active, c.C.dtime};
       g.run();
     }
   }
 }
-template <class R, bool HEAT>
+template <class R, bool HEAT, bool TALL>
 __global__ void __launch_bounds__(BCOL *GR_WAVES) k_gen_reg(const CtxT<R> c, const StateDev old, const StateDev nw) {
   extern __shared__ double lds[];
-  b_gen_reg<R, HEAT>(c, old, nw, bid_here(), lds);
+  b_gen_reg<R, HEAT, TALL>(c, old, nw, bid_here(), lds);
 }
+#define LG_GR_DISPATCH(rk, nl)                   \
+  do {                                           \
+    if ((rk) == 1 && gr_tall(nl)) LG_GR(true, true);   \
+    else if ((rk) == 1) LG_GR(true, false);      \
+    else if (gr_tall(nl)) LG_GR(false, true);    \
+    else LG_GR(false, false);                    \
+  } while (0)
 template <class R>
 void launch_solve_gen(const CtxT<R> &c, const StateDev &old, const StateDev &nw, int rk, hipStream_t st) {
   const int waves = col_waves(c.G);
   if (gen_reg(c.G.nl)) {
     const dim3 g((unsigned)waves), b(BCOL, GR_WAVES);
     const size_t l = gr_lds_bytes(c.G.nl, rk == 1);
-    if (rk == 1)
-      hipLaunchKernelGGL((k_gen_reg<R, true>), g, b, l, st, c, old, nw);
-    else
-      hipLaunchKernelGGL((k_gen_reg<R, false>), g, b, l, st, c, old, nw);
+#define LG_GR(HEAT, TALL) hipLaunchKernelGGL((k_gen_reg<R, HEAT, TALL>), g, b, l, st, c, old, nw)
+    LG_GR_DISPATCH(rk, c.G.nl);
+#undef LG_GR
     return;
   }
   hipLaunchKernelGGL(k_solve_gen<R>, dim3((unsigned)((waves + GEN_GROUPS - 1) / GEN_GROUPS)), dim3(BCOL, NTR * GEN_GROUPS), 0, st, c, old,
@@ -1424,13 +1450,13 @@ __global__ void __launch_bounds__(VS_THREADS, 2)
   b_ver_seg<R, RK, K>(d.c, d.s[a.old_slot], d.s[a.new_slot], bid, lds);
 }
 LG_BATCH_KERNEL(solve_gen, BCOL * NTR * GEN_GROUPS, PH_SOLVE_GEN, b_solve_gen(d.c, d.s[a.old_slot], d.s[a.new_slot], a.rk, bid))
-template <class R, bool HEAT>
+template <class R, bool HEAT, bool TALL>
 __global__ void __launch_bounds__(BCOL *GR_WAVES)
     kb_gen_reg(const MemberDev<R> *__restrict__ M, const int *__restrict__ prefix, int nm, const BatchArgs a) {
   extern __shared__ double lds[];
   Bid bid;
-  const MemberDev<R> &d = batch_block(M, prefix, nm, PH_GEN_REG, bid);
-  b_gen_reg<R, HEAT>(d.c, d.s[a.old_slot], d.s[a.new_slot], bid, lds);
+  const MemberDev<R> &d = batch_block(M, prefix, nm, TALL ? PH_GEN_TALL : PH_GEN_REG, bid);
+  b_gen_reg<R, HEAT, TALL>(d.c, d.s[a.old_slot], d.s[a.new_slot], bid, lds);
 }
 
 template <class R>
@@ -1449,12 +1475,12 @@ bool batch_launch_solve(int ph, dim3 g, dim3 b, hipStream_t st, const MemberDev<
 #undef LG_VS
     return true;
   }
-  if (ph == PH_GEN_REG) {
-    const size_t l = gr_lds_bytes(a.nl_max < GR_MAX_NL ? a.nl_max : GR_MAX_NL, a.rk == 1);
-    if (a.rk == 1)
-      hipLaunchKernelGGL((kb_gen_reg<R, true>), g, b, l, st, M, prefix, nm, a);
-    else
-      hipLaunchKernelGGL((kb_gen_reg<R, false>), g, b, l, st, M, prefix, nm, a);
+  if (ph == PH_GEN_REG || ph == PH_GEN_TALL) {
+    const int lim = ph == PH_GEN_REG ? GR_PART * GR_PARTS : GR_MAX_NL, nl = a.nl_max < lim ? a.nl_max : lim;
+    const size_t l = gr_lds_bytes(nl, a.rk == 1);
+#define LG_GR(HEAT, TALL) hipLaunchKernelGGL((kb_gen_reg<R, HEAT, TALL>), g, b, l, st, M, prefix, nm, a)
+    LG_GR_DISPATCH(a.rk, nl);
+#undef LG_GR
     return true;
   }
   if (ph == PH_SOLVE_GEN) {

@@ -108,15 +108,18 @@ constexpr int GEN_GROUPS = 2;  // 64-column groups per block
 // The tracer solver with the eliminated coefficients in registers and LDS (k_gen_reg): r' of GR_PARTS x GR_PART
 // levels per lane, e' of the GR_EP tracers that have their own, a ring of 2 x gr_k levels of gr_fields values
 // that the tracers share and of heating terms; a wavefront per tracer and one that fills the ring
-constexpr int GR_PART = 16, GR_PARTS = 4, GR_EP = 4, GR_WAVES = NTR + 1;
-__host__ __device__ constexpr int gr_k(bool heat) { return heat ? 2 : 4; }
+constexpr int GR_PART = 16, GR_PARTS = 4, GR_LAST = 8, GR_EP = 4, GR_WAVES = NTR + 1;
+// Columns that fit take it whatever the domain's size; taller ones go through the column scratch (k_solve_gen).
+// Those of more than GR_PARTS parts hold GR_LAST further levels and leave less LDS for the ring.
+constexpr int GR_MAX_NL = GR_PART * GR_PARTS + GR_LAST;
+__host__ __device__ inline bool gen_reg(int nl) { return nl <= GR_MAX_NL; }
+__host__ __device__ inline bool gr_tall(int nl) { return nl > GR_PART * GR_PARTS; }
+__host__ __device__ constexpr int gr_k(bool heat, bool tall) { return (heat ? 2 : 4) / (tall ? 2 : 1); }
 __host__ __device__ constexpr int gr_fields(bool heat) { return heat ? 7 : 5; }
 __host__ __device__ inline size_t gr_lds_bytes(int nl, bool heat) {
-  return sizeof(double) * 64 * ((size_t)GR_EP * nl + 2 * gr_k(heat) * gr_fields(heat) + (heat ? 2 * gr_k(heat) * 5 + 5 : 0));
+  const int ring = 2 * gr_k(heat, gr_tall(nl));
+  return sizeof(double) * 64 * ((size_t)GR_EP * nl + ring * gr_fields(heat) + (heat ? ring * 5 + 5 : 0));
 }
-// Columns that fit take it whatever the domain's size; taller ones go through the column scratch (k_solve_gen).
-constexpr int GR_MAX_NL = GR_PART * GR_PARTS;
-__host__ __device__ inline bool gen_reg(int nl) { return nl <= GR_MAX_NL; }
 template <class R>
 void launch_solve_gen(const CtxT<R> &c, const StateDev &old, const StateDev &nw, int rk, hipStream_t st);
 

@@ -178,9 +178,9 @@ def test_third_order_theta_columns_match_oracle(ny, nx, nl, oro, moist, rows, se
 
 
 @pytest.mark.parametrize("nl,nx", [(3, 5), (4, 63), (5, 64), (16, 65), (17, 7), (18, 7), (31, 128), (33, 129), (48, 9), (50, 9), (63, 64),
-                                   (64, 70)])
+                                   (64, 70), (66, 7), (71, 64), (72, 65)])
 def test_tracer_solver_levels_match_oracle(nl, nx):
-    """The tracer solver keeps up to 64 levels in parts of 16, filled and emptied in chunks of 2 and 4: the
+    """The tracer solver keeps up to 72 levels in parts of 16, worked on in chunks of 1, 2 or 4: the
     smallest columns, the ends of chunks and parts, the tallest column that fits, bitwise against the oracle."""
     cfg = dataclasses.replace(tiny_config(ny=3, nx=nx, n_layers=nl, moist=True), n_oro_layers=max(1, nl - 4))
     g, st = make_case(cfg, cloud_frac=0.3)
@@ -194,7 +194,7 @@ def test_tracer_solver_levels_match_oracle(nl, nx):
 
 
 def test_batched_tracer_solver_with_members_of_different_height():
-    cfgs = [tiny_config(ny=4 + i, nx=30 + 40 * i, n_layers=nl, moist=True) for i, nl in enumerate((66, 7, 64, 70))]
+    cfgs = [tiny_config(ny=4 + i, nx=30 + 40 * i, n_layers=nl, moist=True) for i, nl in enumerate((66, 7, 64, 70, 73))]
     cases = [make_case(c, cloud_frac=0.3) for c in cfgs]
     steps = []
     for c, (g, st) in zip(cfgs, cases):
