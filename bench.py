@@ -67,31 +67,31 @@ SOLVER_BYTES = {"fp64": {1: 152.0, 2: 176.0}, "mixed": {1: 140.0, 2: 164.0}}
 #   theta_v_pert, exner_pert and the new u, v (11 FP64 arrays); theta_v_bg, area_x, area_y, area_z,
 #   volume, slope_x, slope_y, the four horizontal inner-product weights and exner_bg (12 grid
 #   arrays of the form's width); the heating terms (heating_diss, radiation, condensates),
-#   temperature and the six tracer tendencies it updates (10 work arrays); writes the seven density
-#   and the rhotheta_v tendencies (8 work arrays): FP64 88 + 96 + 80 + 64 = 328 B, mixed
-#   88 + 48 + 40 + 32 = 208 B.
-# solve_gen (k_solve_gen, three_band_solver_gen_densities): per tracer the old density, the new
+#   temperature and, in the second substep, the six tracer tendencies it updates (4 and 10 work
+#   arrays, 7 in the mean); writes the seven density and the rhotheta_v tendencies (8 work arrays):
+#   FP64 88 + 96 + 56 + 64 = 304 B, mixed 88 + 48 + 28 + 32 = 196 B.
+# solve_gen (k_gen_reg, three_band_solver_gen_densities): per tracer the old density, the new
 #   density and the tendency read and the new density written (6 x 32 B in FP64), shared per
 #   column old and new w, area_z, volume, the sink velocity of cloud water and the temperature
 #   read and the latent heating written (56 B): 248 B; the mixed form reads the six tendencies,
 #   the temperature and writes the heating at 4 B: 216 B.
 # solve_ver: the mean of the predictor and corrector counts of SOLVER_BYTES.
-KERNEL_BYTES = {"scalar_div": {"fp64": 328.0, "mixed": 208.0}, "solve_gen": {"fp64": 248.0, "mixed": 216.0},
+KERNEL_BYTES = {"scalar_div": {"fp64": 304.0, "mixed": 196.0}, "solve_gen": {"fp64": 248.0, "mixed": 216.0},
                 "solve_ver": {"fp64": 164.0, "mixed": 152.0}}
 KERNEL_NAMES = {"scalar_div": "k_scalar_col (scalar_tend_expl, column-marching)",
-                "solve_gen": "k_solve_gen (three_band_solver_gen_densities, FP64 solve)",
-                "solve_ver": "k_solve_ver (three_band_solver_ver, FP64 solve)"}
+                "solve_gen": "k_gen_reg (three_band_solver_gen_densities, FP64 solve)",
+                "solve_ver": "k_ver_seg (three_band_solver_ver, FP64 solve)"}
 STEP_BYTES = {"dry": 920.0, "moist": 1296.0}  # per grid-point step, whole-step traffic model (FP64)
-# HBM bytes per k_solve_ver dispatch, averaged over predictor and corrector, from two rocprofv3
+# HBM bytes per k_ver_seg dispatch, averaged over predictor and corrector, from two rocprofv3
 # --pmc passes (FETCH_SIZE x 2.0, WRITE_SIZE x 1.0, the factors a 1 GiB device copy gives), per
 # form of the step; profiles/ holds the commands and the per-kernel tables.
-SOLVER_TRAFFIC = {("moist512", "fp64"): 4.369e+09, ("moist512", "mixed"): 4.128e+09}
+SOLVER_TRAFFIC = {("moist512", "fp64"): 3.435e+09, ("moist512", "mixed"): 3.326e+09}
 # the same for the kernels of KERNEL_BYTES, (workload, kernel, form) -> bytes per launch
-KERNEL_TRAFFIC = {("moist512", "solve_ver", "fp64"): 4.369e+09, ("moist512", "solve_ver", "mixed"): 4.128e+09,
-                  ("moist512", "scalar_div", "fp64"): 5.932e+09, ("moist512", "scalar_div", "mixed"): 4.264e+09,
-                  ("moist512", "solve_gen", "fp64"): 5.652e+09, ("moist512", "solve_gen", "mixed"): 5.263e+09}
+KERNEL_TRAFFIC = {("moist512", "solve_ver", "fp64"): 3.435e+09, ("moist512", "solve_ver", "mixed"): 3.326e+09,
+                  ("moist512", "scalar_div", "fp64"): 5.900e+09, ("moist512", "scalar_div", "mixed"): 4.113e+09,
+                  ("moist512", "solve_gen", "fp64"): 3.085e+09, ("moist512", "solve_gen", "mixed"): 2.750e+09}
 # measured HBM bytes per grid-point step of the whole FP64 step (same counters, all kernels)
-STEP_TRAFFIC = {"moist512": 3489.0}
+STEP_TRAFFIC = {"moist512": 2873.0}
 # the reference's own CPU path, flang -O2 -fopenmp on 8 cores, measured on an 8-core Xeon host (the
 # reference tree does not travel, so it cannot be timed beside the GPU)
 REFERENCE_CPU = {"dry128": {"value": 3.19e6, "grid": "129x129x50 dry", "cores": 8},
@@ -153,12 +153,6 @@ def surrogate_mlp():
     return m
 
 
-# the vertical solver's passes per form (1: k_solve_ver, one column per lane; 3: k_ver_rows,
-# k_ver_thomas, k_ver_update on domains with fewer column wavefronts than SIMDs)
-SOLVER_PASSES = {}
-VER_THREE_PASS = "k_ver_rows + k_ver_thomas + k_ver_update (three_band_solver_ver in three passes, FP64 solve)"
-
-
 def make_step(cfg, grid, surface, form, mlp):
     from lgame.config import PREC_FP64, PREC_MIXED, RAD_SURROGATE, RAD_TEACHER
     from lgame.gpu import Step
@@ -169,7 +163,6 @@ def make_step(cfg, grid, surface, form, mlp):
     else:
         c = dataclasses.replace(cfg, precision=PREC_FP64, rad_mode=RAD_TEACHER if cfg.lrad else cfg.rad_mode)
     s = Step(c, grid)
-    SOLVER_PASSES[form] = s.column_passes
     if cfg.lrad:
         s.set_rad_surface(surface)
         if form == "mixed" and MIXED_RAD == "surrogate":
@@ -620,7 +613,7 @@ def main():
         name = max(ks, key=lambda k: ks[k][0])
         ms, n = ks[name]
         b = KERNEL_BYTES.get(name, {}).get(form)
-        kname = VER_THREE_PASS if name == "solve_ver" and SOLVER_PASSES.get(form) == 3 else KERNEL_NAMES.get(name, name)
+        kname = KERNEL_NAMES.get(name, name)
         out_r = {"kernel": f"{kname} of the {form} form", "bound": "hbm", "peak": HBM_PEAK_GBS,
                  "unit": "GB/s", "ms_per_step": ms, "launches_per_step": n, "avg_launch_us": 1e3 * ms / max(n, 1),
                  "share_of_step": ms / (1e3 * res[form][0] / args.steps)}
@@ -679,8 +672,7 @@ def main():
                   for f, r in res.items()},
         "roofline": kernel_roofline(head),
         "roofline_solver_ver": {
-            "kernel": (f"{VER_THREE_PASS if SOLVER_PASSES.get(rf) == 3 else 'k_solve_ver (three_band_solver_ver, FP64 solve)'}"
-                       f", both substeps, of the {rf} form"),
+            "kernel": f"k_ver_seg (three_band_solver_ver, FP64 solve), both substeps, of the {rf} form",
             "bound": "hbm",
             "achieved": solver_gbs,
             "peak": HBM_PEAK_GBS,

@@ -465,12 +465,15 @@ int lgame_profile_reset(lgame_handle *h);
  * diff_coef, diff_dual, diff_mom, diff_flux, diff_div (the last six run only with diffusion).
  * The scalar fluxes are formed inside the scalar divergence kernel, the mass fluxes and the
  * kinetic energy inside the potential-vorticity kernel, the kinetic-energy gradient inside the
- * vorticity-flux kernel and the full theta_v of the third-order theta where it is loaded, so the
- * theta_fill, mass_flux, scalar_flux, ke and ke_grad entries are kept for the order but not used.  The pgrad entry is the first substep's
- * pressure gradient together with its wind update, vec_tend the second substep's wind update.
- * The scalar divergence kernel marches down the columns; its
- * levels can be cut into 1, 2, 4 or 8 segments (at least 4 levels each) so that small domains
- * fill the GPU: lgame_init picks the segments that give about four wavefronts per SIMD,
+ * vorticity-flux kernel, the full theta_v of the third-order theta where it is loaded, its gradient
+ * inside its divergence kernel (theta_div), the Klemp dissipation alone inside the temperature kernel,
+ * and the diffusive fluxes and their divergence in one kernel (diff_flux), so the theta_fill,
+ * theta_grad, mass_flux, scalar_flux, ke, ke_grad and diff_div entries are kept for the order but not
+ * used.  The pgrad entry is the first substep's pressure gradient together with its wind update,
+ * vec_tend the second substep's wind update.
+ * The scalar divergence, theta_div and diff_flux kernels march down the columns; their levels can
+ * be cut into 1, 2, 4 or 8 segments (at least 4 levels each) so that small domains fill the GPU:
+ * lgame_init picks the segments that give about four wavefronts per SIMD,
  * lgame_autotune times 1, 2, 4 and 8 after the block shapes, lgame_set_segments sets them and
  * lgame_get_segments reads the choice.  Every choice gives the same bits. */
 #define LGAME_N_TILES 21
@@ -478,12 +481,14 @@ int lgame_autotune(lgame_handle *h, int steps, int *rows);
 int lgame_set_tiles(lgame_handle *h, const int *rows);
 int lgame_set_segments(lgame_handle *h, int nseg);
 int lgame_get_segments(lgame_handle *h, int *nseg);
-/* The implicit vertical solver (three_band_solver_ver, mo_column_solvers.F90:21-351) runs in one
+/* The implicit vertical solver (three_band_solver_ver, mo_column_solvers.F90:21-351) holds a column
+ * of up to 72 layers in registers and on-chip memory, in one kernel.  Taller columns go in one
  * pass per column (one lane a column) or in three passes: the rows of the system and the new
- * state by one thread per (column, level), the Thomas recursion alone per column.  lgame_init
+ * state by one thread per (column, level), the Thomas recursion alone per column, and the calls
+ * below choose between these two (for the others they only set and read the value).  lgame_init
  * picks three passes when the domain has fewer than 1024 wavefronts of 64 columns (fewer than the
- * GPU's SIMDs) and at least 3 layers, one pass otherwise; lgame_autotune times both on domains of
- * fewer than 2048 such wavefronts and keeps the faster; lgame_set_column_passes (1 or 3) sets it
+ * GPU's SIMDs) and at least 3 layers, one pass otherwise; lgame_autotune times both for taller
+ * columns on domains of fewer than 2048 such wavefronts and keeps the faster; lgame_set_column_passes (1 or 3) sets it
  * and lgame_get_column_passes reads it.  Both give the same bits.  No reference counterpart. */
 int lgame_set_column_passes(lgame_handle *h, int passes);
 int lgame_get_column_passes(lgame_handle *h, int *passes);
