@@ -1,5 +1,8 @@
 // lgame_solve.hip -- implicit vertical column solvers of the HEVI step (FP64 in both forms, gfx950).
 //
+// Columns of up to 72 layers stay on the chip between the elimination and the back substitution
+// (k_ver_seg, k_gen_reg).  The kernels for taller ones (k_solve_ver and its three-pass form, k_solve_gen)
+// work as follows, and the others take their expressions.
 // One column per lane: consecutive lanes take consecutive x, so every per-level load and store
 // of a wavefront is one coalesced 512-byte row segment.  The tridiagonal coefficients of a
 // column are built while streaming down the column with a rolling window of three layers; the

@@ -306,7 +306,7 @@ class Step:
 
     @property
     def column_passes(self) -> int:
-        """The vertical solver in one pass per column (1) or in three passes (3)."""
+        """The vertical solver of columns of over 72 layers in one pass per column (1) or in three passes (3)."""
         n = ctypes.c_int(0)
         self._check(self.lib.lgame_get_column_passes(self.h, ctypes.byref(n)), "lgame_get_column_passes")
         return n.value
