@@ -404,13 +404,16 @@ __device__ __forceinline__ void b_theta_col(const CtxT<R> &c, const StateDev &st
   }
   R az_up = R(0.0);  // upper interface area and volume of the unfinished cell
   Inv<R> V_up(R(1.0));
-  for (int m = m0; m <= l1 + 1; ++m) {  // (at m = n_layers+1 only the lowest cell is finished)
-    const bool terr = m > nflat;
+  // layer m: its gradients, and the cell above it.  The flat layers have no terrain terms: they are not
+  // formed, rather than multiplied by zero, so that the slopes stored there are not used and a value that
+  // is not finite stays in its layer, as in div_h and grad_hor.
+  auto layer = [&](auto terrain, int m) {
+    constexpr bool TERR = decltype(terrain)::value;
     const int ml = m < nl ? m : nl;  // (below the lowest layer, its own values once more)
     const ix_t iC = LG_IX(G, p.ji, p.js, ml), iN = LG_IX(G, p.jmr, p.js, ml), iS = LG_IX(G, p.j1, p.js, ml);
     const ix_t iM = LG_IX(G, p.ji, p.jkm, ml), iMs = LG_IX(G, p.ji + 1, p.jkm, ml);
     const ix_t dl = ml < nl ? (ix_t)G.lvl : 0;
-    // all loads of the layer, issued before any is used
+    // all loads of the layer, issued before any is used (what a flat layer does not use is not loaded)
     R nc[NF], nn[NF], ns[NF];
     fld(iC + dl, nc);
     fld(iN + dl, nn);
@@ -419,38 +422,41 @@ __device__ __forceinline__ void b_theta_col(const CtxT<R> &c, const StateDev &st
     const R dzc_ = c.g.dz[iC + dl], dzn_ = c.g.dz[iN + dl], dzs_ = c.g.dz[iS + dl];
     const R p4c = c.g.ipw[4][iC], p4n = c.g.ipw[4][iN], p4s = c.g.ipw[4][iS];
     const R p5c = c.g.ipw[5][iC], p5n = c.g.ipw[5][iN], p5s = c.g.ipw[5][iS];
-    const R sxm = c.g.slope_x[iM], sym = c.g.slope_y[iM], syms = c.g.slope_y[iMs];
+    const R sx = c.g.slope_x[iM], syn = c.g.slope_y[iM], sys = c.g.slope_y[iMs];
     const R ax0 = c.g.area_x[iM], ay0 = c.g.area_y[iM], ay1 = c.g.area_y[iMs];
     const R az = c.g.area_z[iC], vol = c.g.volume[iC];
     const R w0 = c.g.ipw[0][iM], w1 = c.g.ipw[1][iM], w2 = c.g.ipw[2][iM], w3 = c.g.ipw[3][iM];
     __builtin_amdgcn_sched_barrier(0);
     const Inv<R> dx(dx_), dyn(dyn_), dys(dys_), dzc(dzc_), dzn(dzn_), dzs(dzs_);
-    const VccGeo<R> geo{from_next_lane(sxm), sym, sxm, syms, w0, w1, w2, w3};
+    const VccGeo<R> geo{from_next_lane(sx), syn, sx, sys, w0, w1, w2, w3};
     const R ax1 = from_next_lane(ax0), p4w = from_prev_lane(p4c), p5w = from_prev_lane(p5c);
-    // the areas of the interfaces of the cell above that carry a contravariant correction and the slopes
-    // of the terrain-following layers, zero for the others (no branches below)
-    const int jl = m - 1;
-    const R az0 = jl > nflat ? az_up : R(0.0), az1 = jl >= nflat && jl < nl ? az : R(0.0);
-    const R sx = terr ? sxm : R(0.0), syn = terr ? sym : R(0.0), sys = terr ? syms : R(0.0);
+    const R az1 = m <= nl ? az : R(0.0);  // no correction at the surface
     const bool st_cell = p.cell && m > l0;
     const ix_t iF = LG_IX(G, p.ji, p.js, m > 1 ? m - 1 : 1);
 #pragma unroll
     for (int q = 0; q < NF; ++q) {
       ThetaField<R> &f = F[q];
       const R vc1 = (f.c - nc[q]) / dzc, vn1 = (f.n - nn[q]) / dzn, vs1 = (f.s - ns[q]) / dzs;
-      const R w = from_prev_lane(f.c), vw = from_prev_lane(f.vc), vw1 = from_prev_lane(vc1);
-      // grad_hor with remap_ver2hor_x/_y, mo_averaging.F90:56-136
-      const R gx = (f.c - w) / dx - sx * (R(0.5) * (p4w * vw + p4c * f.vc + p5w * vw1 + p5c * vc1));
-      const R gn = (f.n - f.c) / dyn - syn * (R(0.5) * (p4n * f.vn + p4c * f.vc + p5n * vn1 + p5c * vc1));
-      const R gs = (f.c - f.s) / dys - sys * (R(0.5) * (p4c * f.vc + p4s * f.vs + p5c * vc1 + p5s * vs1));
+      const R w = from_prev_lane(f.c);
+      R gx = (f.c - w) / dx, gn = (f.n - f.c) / dyn, gs = (f.c - f.s) / dys;
+      if (TERR) {  // grad_hor with remap_ver2hor_x/_y, mo_averaging.F90:56-136
+        const R vw = from_prev_lane(f.vc), vw1 = from_prev_lane(vc1);
+        gx = gx - sx * (R(0.5) * (p4w * vw + p4c * f.vc + p5w * vw1 + p5c * vc1));
+        gn = gn - syn * (R(0.5) * (p4n * f.vn + p4c * f.vc + p5n * vn1 + p5c * vc1));
+        gs = gs - sys * (R(0.5) * (p4c * f.vc + p4s * f.vs + p5c * vc1 + p5s * vs1));
+      }
       const Faces<R> fc{from_next_lane(gx), gn, gx, gs};
-      const R I = vcc_sub(f.P, geo, fc);
-      const R d = (f.hh + (f.I * az0 - I * az1)) / V_up;
+      R d;
+      if (TERR) {  // (f.I and f.P are zero below the flat layers: interface nflat+1 has no terms of the layer above it)
+        const R I = vcc_sub(f.P, geo, fc);
+        d = (f.hh + (f.I * az_up - I * az1)) / V_up;
+        f.P = vcc_sub(R(0.0), geo, fc);
+        f.I = I;
+      } else {
+        d = f.hh / V_up;
+      }
       if (st_cell) c.w.tfd[q][iF] = d;
       f.hh = fc.e * ax1 + fc.n * ay0 - fc.w * ax0 - fc.s * ay1;
-      f.P = vcc_sub(R(0.0), geo, fc);
-      if (m <= nflat) f.P = R(0.0);  // interface nflat+1 has no terms of the layer above it
-      f.I = I;
       f.c = nc[q];
       f.n = nn[q];
       f.s = ns[q];
@@ -460,7 +466,12 @@ __device__ __forceinline__ void b_theta_col(const CtxT<R> &c, const StateDev &st
     }
     az_up = az;
     V_up = Inv<R>(vol);
-  }
+  };
+  // (at m = n_layers+1 only the lowest cell is finished)
+  const int last = l1 + 1, flat = nflat < nl && nflat < last ? nflat : last;
+  int m = m0;
+  for (; m <= flat; ++m) layer(std::false_type{}, m);
+  for (; m <= last; ++m) layer(std::true_type{}, m);
 }
 template <class R, int NF>
 __global__ void __launch_bounds__(BX * 4) k_theta_col(const CtxT<R> c, const StateDev s, int nseg) {

@@ -203,6 +203,57 @@ def test_check_finite_flags_injected_nan():
     assert g.count_nonfinite(1) == 2
 
 
+FLAT = dataclasses.replace(tiny_config(ny=9, nx=20, n_layers=16), n_oro_layers=6)  # levels 1..10 are flat
+FLAT_CASES = {
+    "theta_o3": dataclasses.replace(FLAT, theta_adv_order=3),
+    "moist_theta_o3": dataclasses.replace(FLAT, theta_adv_order=3, lmoist=True),
+}
+
+
+@pytest.mark.parametrize("name", list(FLAT_CASES))
+@pytest.mark.parametrize("level", [2, 4, 10, 11, 16])
+def test_non_finite_values_reach_the_same_points_as_in_the_oracle(name, level):
+    """One theta_v perturbation that is not a number, in a flat or a terrain-following layer: after one
+    and two steps the same points of every field are not finite as in the oracle, which does not form
+    the terrain terms of the flat layers."""
+    cfg = FLAT_CASES[name]
+    grid, st = make_case(cfg, cloud_frac=0.2 if cfg.lmoist else 0.0)
+    bad = {k: v.copy() for k, v in st.items()}
+    bad["theta_v_pert"][4, 10, level - 1] = np.nan
+    g = Step(cfg, grid)
+    g.start(bad)
+    o = CpuOracle(cfg, grid)
+    o.start(bad)
+    for n in (1, 2):
+        g.run(n - 1, 1)
+        o.run(n - 1, 1)
+        got, want = g.get_state(n % 2), o.get_state(n % 2)
+        for k in want:
+            assert np.array_equal(np.isfinite(got[k]), np.isfinite(want[k])), (k, n)
+    g.close()
+
+
+@pytest.mark.parametrize("name", list(FLAT_CASES))
+def test_slopes_of_flat_layers_are_not_used(name):
+    """A grid whose slopes in the flat layers are not numbers gives the oracle's bits."""
+    cfg = FLAT_CASES[name]
+    grid, st = make_case(cfg, cloud_frac=0.2 if cfg.lmoist else 0.0)
+    holes = dict(grid)
+    for k in ("slope_x", "slope_y"):
+        holes[k] = grid[k].copy()
+        holes[k][:, :, :cfg.n_layers - cfg.n_oro_layers] = np.nan
+    g = Step(cfg, holes)
+    g.start(st)
+    g.run(0, 3)
+    got = g.get_state(1)
+    g.close()
+    o = CpuOracle(cfg, grid)
+    o.start(st)
+    o.run(0, 3)
+    want = o.get_state(1)
+    assert all(np.array_equal(got[k], want[k]) for k in want)
+
+
 def test_step_argument_errors():
     cfg = tiny_config()
     grid, st = make_case(cfg)
