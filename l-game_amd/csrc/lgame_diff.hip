@@ -293,7 +293,7 @@ __global__ void __launch_bounds__(BX * BY) k_diff_mom(const CtxT<R> c, const Sta
 // upper interface for all fields of a layer, and finishes the cell above, which only waited for this
 // layer's contravariant correction and vertical flux.  The fluxes never go to memory: as two kernels
 // with 24 flux fields in between (moist) it moved 723 B per cell in FP64 where 264 are needed.
-// It is bound by its instructions now, one wavefront per SIMD in FP64 (390 registers, 12,900 cycles a
+// It is bound by its instructions now, one wavefront per SIMD in FP64 (380 registers, 12,900 cycles a
 // layer): eight quotients per field and cell, which share seven denominators, and no branches in the
 // field loop (with them 526 us in FP64).  Both kernels before -> this one, us: 256x256x60 FP64 759 -> 456,
 // 321x225x51 mixed 482 -> 248.
@@ -417,17 +417,18 @@ __device__ __forceinline__ void b_diff_col(const CtxT<R> &c, const StateDev &st,
     x.vs = c.w.visc[iS];
     x.kv = c.w.kv[iC];
   };
-  In x;
-  for (int m = m0; m <= l1 + 1; ++m) {  // (at m = n_layers+1 only the lowest cell is finished)
-    const bool terr = m > nflat;
+  // layer m: its fluxes, and the cell above it.  The flat layers have no terrain terms: they are not formed,
+  // rather than multiplied by zero (as in k_theta_col; and so with the vertical fluxes that are off).
+  auto layer = [&](auto terrain, int m) {
+    constexpr bool TERR = decltype(terrain)::value;
     // A layer's loads are issued together, before any is used: left to itself the compiler loads field by
     // field and waits for each (792 us instead of 571 in the form measured above with branches).
+    In x;
     load(m, x);
     __builtin_amdgcn_sched_barrier(0);
     const Inv<R> dx(x.dx), dyn(x.dyn), dys(x.dys), dzc(x.dzc), dzn(x.dzn), dzs(x.dzs);
     const VccGeo<R> geo{from_next_lane(x.sxm), x.sym, x.sxm, x.syms, x.w0, x.w1, x.w2, x.w3};
     const R p4c = x.p4c, p4n = x.p4n, p4s = x.p4s, p5c = x.p5c, p5n = x.p5n, p5s = x.p5s;
-    const R sx = terr ? x.sx : R(0.0), syn = terr ? x.syn : R(0.0), sys = terr ? x.sys : R(0.0);
     const R ax0 = x.ax, ay0 = x.ayn, ay1 = x.ays, az = x.az, vol = x.vol, v_c = x.vc, v_n = x.vn, v_s = x.vs, kv = x.kv;
     const R ax1 = from_next_lane(ax0), p4w = from_prev_lane(p4c), p5w = from_prev_lane(p5c);
     // coefficients at the west, north and south face and the upper interface
@@ -438,7 +439,7 @@ __device__ __forceinline__ void b_diff_col(const CtxT<R> &c, const StateDev &st,
       ctx = R(0.5) * (from_prev_lane(k_c) + k_c);
       ctn = R(0.5) * (k_n + k_c);
       cts = R(0.5) * (k_c + k_s);
-      ctw = lvt && inner ? R(0.5) * (a_up + a) : R(0.0);
+      ctw = R(0.5) * (a_up + a);
       a_up = a;
     }
     if (MASS) {
@@ -446,17 +447,13 @@ __device__ __forceinline__ void b_diff_col(const CtxT<R> &c, const StateDev &st,
       cmx = R(0.5) * (from_prev_lane(k_c) + k_c);
       cmn = R(0.5) * (k_n + k_c);
       cms = R(0.5) * (k_c + k_s);
-      cmw = lvm && inner ? R(0.5) * (kv_up + kv) : R(0.0);
+      cmw = R(0.5) * (kv_up + kv);
     }
     kv_up = kv;
     g_c = x.gc;
     g_n = x.gn;
     g_s = x.gs;
-    // The cell above lies among the flat or the terrain-following layers: the areas of its interfaces
-    // that carry a contravariant correction, zero for the others, so that the fields need no branch (as
-    // the slopes, zero in the flat layers; the gradient at the bottom is a difference of equal values)
-    const int jl = m - 1;
-    const R az0 = jl > nflat ? az_up : R(0.0), az1 = jl >= nflat && jl < nl ? az : R(0.0);
+    const R az1 = m <= nl ? az : R(0.0);  // no contravariant correction at the surface
     const bool st_cell = p.cell && m > l0;
     const ix_t iF = LG_IX(G, p.ji, p.js, m > 1 ? m - 1 : 1);
 #pragma unroll
@@ -465,20 +462,27 @@ __device__ __forceinline__ void b_diff_col(const CtxT<R> &c, const StateDev &st,
       const bool T = TEMP && q == 0;
       // vertical gradients at the lower interface of the layer
       const R vc1 = (f.c - x.nc[q]) / dzc, vn1 = (f.n - x.nn[q]) / dzn, vs1 = (f.s - x.ns[q]) / dzs;
-      const R w = from_prev_lane(f.c), vw = from_prev_lane(f.vc), vw1 = from_prev_lane(vc1);
-      // grad_hor with remap_ver2hor_x/_y, mo_averaging.F90:56-136
-      const R gx = (f.c - w) / dx - sx * (R(0.5) * (p4w * vw + p4c * f.vc + p5w * vw1 + p5c * vc1));
-      const R gn = (f.n - f.c) / dyn - syn * (R(0.5) * (p4n * f.vn + p4c * f.vc + p5n * vn1 + p5c * vc1));
-      const R gs = (f.c - f.s) / dys - sys * (R(0.5) * (p4c * f.vc + p4s * f.vs + p5c * vc1 + p5s * vs1));
+      const R w = from_prev_lane(f.c);
+      R gx = (f.c - w) / dx, gn = (f.n - f.c) / dyn, gs = (f.c - f.s) / dys;
+      if (TERR) {  // grad_hor with remap_ver2hor_x/_y, mo_averaging.F90:56-136 (at the bottom a difference of equal values)
+        const R vw = from_prev_lane(f.vc), vw1 = from_prev_lane(vc1);
+        gx = gx - x.sx * (R(0.5) * (p4w * vw + p4c * f.vc + p5w * vw1 + p5c * vc1));
+        gn = gn - x.syn * (R(0.5) * (p4n * f.vn + p4c * f.vc + p5n * vn1 + p5c * vc1));
+        gs = gs - x.sys * (R(0.5) * (p4c * f.vc + p4s * f.vs + p5c * vc1 + p5s * vs1));
+      }
       const R fx = (T ? ctx : cmx) * gx, fn = (T ? ctn : cmn) * gn, fs = (T ? cts : cms) * gs;
       const Faces<R> fc{from_next_lane(fx), fn, fx, fs};
-      const R I = vcc_sub(f.P, geo, fc);
-      const R dw = (T ? ctw : cmw) * f.vc;
-      const R d = (f.hh + (f.I * az0 - I * az1)) / V_up + (f.dw * az_up - dw * az) / V_up;
+      const R dw = (T ? lvt : lvm) && inner ? (T ? ctw : cmw) * f.vc : R(0.0);
+      R hor = f.hh;
+      if (TERR) {  // (f.I and f.P are zero below the flat layers: interface nflat+1 has no terms of the layer above it)
+        const R I = vcc_sub(f.P, geo, fc);
+        hor = hor + (f.I * az_up - I * az1);
+        f.P = vcc_sub(R(0.0), geo, fc);
+        f.I = I;
+      }
+      const R d = hor / V_up + (f.dw * az_up - dw * az) / V_up;
       if (st_cell) (T ? c.w.tdh : c.w.mdt[q - Q0])[iF] = d;
       f.hh = fc.e * ax1 + fc.n * ay0 - fc.w * ax0 - fc.s * ay1;
-      f.P = vcc_sub(R(0.0), geo, fc);
-      f.I = I;
       f.dw = dw;
       f.c = x.nc[q];
       f.n = x.nn[q];
@@ -487,12 +491,14 @@ __device__ __forceinline__ void b_diff_col(const CtxT<R> &c, const StateDev &st,
       f.vn = vn1;
       f.vs = vs1;
     }
-    if (m <= nflat)  // the correction of interface nflat+1 has no terms of the layer above it
-#pragma unroll
-      for (int q = 0; q < NF; ++q) F[q].P = R(0.0);
     az_up = az;
     V_up = Inv<R>(vol);
-  }
+  };
+  // (at m = n_layers+1 only the lowest cell is finished)
+  const int last = l1 + 1, flat = nflat < nl && nflat < last ? nflat : last;
+  int m = m0;
+  for (; m <= flat; ++m) layer(std::false_type{}, m);
+  for (; m <= last; ++m) layer(std::true_type{}, m);
 }
 
 template <class R, bool TR, bool TEMP, bool MASS>

@@ -233,10 +233,33 @@ def test_non_finite_values_reach_the_same_points_as_in_the_oracle(name, level):
     g.close()
 
 
-@pytest.mark.parametrize("name", list(FLAT_CASES))
+@pytest.mark.parametrize("vertical", [True, False])
+@pytest.mark.parametrize("level", [2, 4, 10, 11, 16])
+def test_non_finite_diffusive_heating_matches_oracle(level, vertical):
+    """The same with a gas density and a temperature that are not numbers, for the heating rate of the
+    temperature diffusion, with and without its vertical part."""
+    cfg = diff(FLAT, ltemp_diff_v=vertical)
+    grid, st = make_case(cfg)
+    for field in ("rho", "theta_v_pert"):
+        bad = {k: v.copy() for k, v in st.items()}
+        bad[field][4, 10, level - 1] = np.nan
+        g = Step(cfg, grid)
+        g.start(bad)
+        g.run(0, 1)
+        got = g.diag("temp_diff_heating")
+        g.close()
+        o = CpuOracle(cfg, grid)
+        o.start(bad)
+        o.run(0, 1)
+        want = o.get_diag("temp_diff_heating", got.shape)
+        assert not np.isfinite(want).all() and np.isfinite(want).any()
+        assert np.array_equal(np.isfinite(got), np.isfinite(want)), field
+
+
+@pytest.mark.parametrize("name", [*FLAT_CASES, "diff", "moist_diff"])
 def test_slopes_of_flat_layers_are_not_used(name):
     """A grid whose slopes in the flat layers are not numbers gives the oracle's bits."""
-    cfg = FLAT_CASES[name]
+    cfg = FLAT_CASES[name] if name in FLAT_CASES else diff(FLAT, lmoist=name == "moist_diff")
     grid, st = make_case(cfg, cloud_frac=0.2 if cfg.lmoist else 0.0)
     holes = dict(grid)
     for k in ("slope_x", "slope_y"):
