@@ -320,7 +320,7 @@ int enqueue_pchevi(const CtxT<R> &c, const StateDev &old, const StateDev &nw, in
     launch_theta_col(c, s, nfield, tiles.by[KI_THETA_DIV], tiles.seg, st);
     if (pk) prof->end(PROF_KERNEL0 + KI_THETA_DIV);
   };
-  LG_LAUNCH(KI_TEMPERATURE, k_temperature, nx, ny, nl, c, old);
+  LG_LAUNCH(KI_TEMPERATURE, k_temperature, nx, ny, nl, c, old, 1);
   // update_sfc_turb_quantities with state_old (mo_manage_pchevi.F90:52-54)
   if (c.C.lsfc_turb) LG_LAUNCH(KI_DIFF_DUAL, k_sfc_turb, nx, ny, 1, c, old);
   // update_rad_fluxes with state_old (mo_manage_pchevi.F90:56-58)
@@ -1141,9 +1141,9 @@ int lgame_integrals(lgame_handle *h, int slot, double *out) {
   if (!h->stepped) {  // before the first step the temperature is diagnosed from this state (control.F90:484)
     const Geom &G = h->c.G;
     if (h->mixed)
-      hipLaunchKernelGGL(k_temperature<float>, grid3(G.nx, G.ny, G.nl), dim3(BX, BY, 1), 0, h->stream, h->cf, h->slot[slot]);
+      hipLaunchKernelGGL(k_temperature<float>, grid3(G.nx, G.ny, G.nl), dim3(BX, BY, 1), 0, h->stream, h->cf, h->slot[slot], 0);
     else
-      hipLaunchKernelGGL(k_temperature<double>, grid3(G.nx, G.ny, G.nl), dim3(BX, BY, 1), 0, h->stream, h->c, h->slot[slot]);
+      hipLaunchKernelGGL(k_temperature<double>, grid3(G.nx, G.ny, G.nl), dim3(BX, BY, 1), 0, h->stream, h->c, h->slot[slot], 0);
   }
   if (h->mixed)
     hipLaunchKernelGGL(k_integrals<float>, dim3(RED_GRID), dim3(RED_BLOCK), 0, h->stream, h->c, h->slot[slot],
@@ -1993,10 +1993,10 @@ int lgame_rad_columns(lgame_handle *h, int slot, double t, float *x, float *y) {
   RadDev r = rad_dev(h);
   const dim3 gc((unsigned)((ncol + BCOL - 1) / BCOL)), bc(BCOL);
   if (h->mixed) {
-    hipLaunchKernelGGL(k_temperature<float>, grid3(G.nx, G.ny, G.nl), dim3(BX, BY, 1), 0, h->stream, h->cf, h->slot[slot]);
+    hipLaunchKernelGGL(k_temperature<float>, grid3(G.nx, G.ny, G.nl), dim3(BX, BY, 1), 0, h->stream, h->cf, h->slot[slot], 0);
     hipLaunchKernelGGL(k_rad<float>, gc, bc, 0, h->stream, h->cf, h->slot[slot], r, t, RAD_X | RAD_Y);
   } else {
-    hipLaunchKernelGGL(k_temperature<double>, grid3(G.nx, G.ny, G.nl), dim3(BX, BY, 1), 0, h->stream, h->c, h->slot[slot]);
+    hipLaunchKernelGGL(k_temperature<double>, grid3(G.nx, G.ny, G.nl), dim3(BX, BY, 1), 0, h->stream, h->c, h->slot[slot], 0);
     hipLaunchKernelGGL(k_rad<double>, gc, bc, 0, h->stream, h->c, h->slot[slot], r, t, RAD_X | RAD_Y);
   }
   HIPCHK(h, hipGetLastError());

@@ -6,7 +6,9 @@
 
 namespace lgame {
 
-template <class R> __global__ void k_temperature(const CtxT<R> c, const StateDev s);
+// diss: the step's own call, which also forms the dissipation rate of the Klemp layer (klemp_only); the calls that
+// diagnose the temperature of a slot between steps leave the last step's rate as it is
+template <class R> __global__ void k_temperature(const CtxT<R> c, const StateDev s, int diss);
 template <class R> __global__ void k_theta_edge(const CtxT<R> c, const StateDev s, int nfield);
 // the potential vorticity, the mass fluxes and (with_ke) the kinetic energy
 template <class R> __global__ void k_pot_vort(const CtxT<R> c, const StateDev s, int with_ke);

@@ -51,7 +51,7 @@ __device__ __forceinline__ R klemp_heating(const CtxT<R> &c, const StateDev &s, 
 // (mo_p_grad.F90:106-120) and the sink velocity of cloud water, which depends only on this state
 // and the temperature (the generalized-density solver of both substeps reads it).
 template <class R>
-__device__ __forceinline__ void b_temperature(const CtxT<R> &c, const StateDev &s, const Bid bid) {
+__device__ __forceinline__ void b_temperature(const CtxT<R> &c, const StateDev &s, int diss, const Bid bid) {
   KIDX;
   if (jk > c.G.nx || ji > c.G.ny || jl > c.G.nl) return;
   const ix_t i = LG_IX(c.G, ji, jk, jl);
@@ -68,11 +68,11 @@ __device__ __forceinline__ void b_temperature(const CtxT<R> &c, const StateDev &
   }
   // simple_dissipation_rate with the Klemp layer alone: a product of this cell's values (with a
   // friction of the wind it follows the momentum diffusion, k_dissipation)
-  if (klemp_only(c) && jl <= diss_levels(c)) c.w.heating_diss[i] = klemp_heating(c, s, ji, jk, jl, R(0.0), R(0.0), rs);
+  if (diss && klemp_only(c) && jl <= diss_levels(c)) c.w.heating_diss[i] = klemp_heating(c, s, ji, jk, jl, R(0.0), R(0.0), rs);
 }
 template <class R>
-__global__ void __launch_bounds__(BX * BY) k_temperature(const CtxT<R> c, const StateDev s) {
-  b_temperature(c, s, bid_here());
+__global__ void __launch_bounds__(BX * BY) k_temperature(const CtxT<R> c, const StateDev s, int diss) {
+  b_temperature(c, s, diss, bid_here());
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -801,7 +801,7 @@ __global__ void __launch_bounds__(BX * BY) k_vort_flux_vt(const CtxT<R> c, const
 
 // The plain form (FP64 stencils) and the mixed form (FP32 stencils).
 #define LG_INSTANTIATE(R)                                                                                  \
-  template __global__ void k_temperature<R>(const CtxT<R>, const StateDev);                              \
+  template __global__ void k_temperature<R>(const CtxT<R>, const StateDev, int);                         \
   template __global__ void k_theta_edge<R>(const CtxT<R>, const StateDev, int);                          \
   template __global__ void k_pot_vort<R>(const CtxT<R>, const StateDev, int);                            \
   template __global__ void k_pot_vort2<R>(const CtxT<R>, const StateDev, int);                           \
@@ -816,7 +816,7 @@ LG_INSTANTIATE(float)
 #undef LG_INSTANTIATE
 
 // ---- the same kernels over a group of domains (one launch per phase) ------------------------
-LG_BATCH_KERNEL(temperature, BX * BY, PH_TEMPERATURE, b_temperature(d.c, d.s[a.old_slot], bid))
+LG_BATCH_KERNEL(temperature, BX * BY, PH_TEMPERATURE, b_temperature(d.c, d.s[a.old_slot], 1, bid))
 LG_BATCH_KERNEL(theta_edge, BX * BY, PH_THETA_EDGE, b_theta_edge(d.c, d.s[a.state_slot], a.nfield, bid))
 LG_BATCH_KERNEL(pgrad, BX * BY, PH_PGRAD, b_pgrad_vt(d.c, d.s[a.old_slot], d.s[a.new_slot], a.lfirst, bid))
 LG_BATCH_KERNEL(pot_vort, BX * BY, PH_POT_VORT, b_pot_vort(d.c, d.s[a.state_slot], a.ke, bid))

@@ -14,7 +14,7 @@ import pytest
 
 from lgame import surrogate
 from lgame.cases import make_case, moist3d_config, radiation_surface, schaer_config, tiny_config
-from lgame.config import PREC_MIXED, RAD_SURROGATE, RAD_TEACHER
+from lgame.config import PREC_FP64, PREC_MIXED, RAD_SURROGATE, RAD_TEACHER
 from lgame.gpu import LgameError, Step
 
 pytestmark = pytest.mark.gpu
@@ -149,3 +149,34 @@ def test_checkpoint_pressure_gradient_parts_are_summed():
     got = b.get_state(1)
     b.close()
     assert all(np.array_equal(got[f], want[f]) for f in want)
+
+
+@pytest.mark.parametrize("precision", [PREC_FP64, PREC_MIXED])
+def test_diagnosing_a_slot_keeps_the_carried_fields(precision):
+    """Reading the radiation columns of either slot between steps, or the budget sums of a restored run
+    before its first step, diagnoses the temperature of that slot and nothing that a run carries: the last
+    step's dissipation rate (of the Klemp layer alone) and the checkpoint stay as they are."""
+    cfg = dataclasses.replace(tiny_config(ny=7, nx=9, n_layers=12, moist=True), lrad=True, rad_mode=RAD_TEACHER, dtime_rad=6.0,
+                              precision=precision)
+    g, st = make_case(cfg, cloud_frac=0.02)
+    a = Step(cfg, g)
+    a.start(st)
+    a.set_rad_surface(radiation_surface(cfg, g, st))
+    a.run(0, 5, t_init=T0)
+    rate, blob = a.diag("heating_diss"), a.checkpoint()
+    assert np.abs(rate).max() > 0.0
+    for slot in (0, 1):
+        a.rad_columns(slot, T0)
+        assert np.array_equal(a.diag("heating_diss"), rate)
+    assert a.checkpoint() == blob
+    b = Step(cfg, g)
+    b.set_rad_surface(radiation_surface(cfg, g, st))
+    for slot in (0, 1):
+        b.set_state(slot, a.get_state(slot))
+    b.restore(blob)
+    for slot in (0, 1):
+        b.integrals(slot)
+    assert np.array_equal(b.diag("heating_diss"), rate)
+    assert b.checkpoint() == blob
+    a.close()
+    b.close()
