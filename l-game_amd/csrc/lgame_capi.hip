@@ -1307,9 +1307,12 @@ int lgame_checkpoint_load(lgame_handle *h, const void *buf, long long bytes) {
   // the dissipation rate is formed (and read) in its levels only
   auto zero_below = [&](const auto &c) {
     const size_t es = sizeof(*c.w.heating_diss.p), n = (size_t)diss_levels(c) * (size_t)c.G.lvl;
-    return hipMemset((char *)c.w.heating_diss.p + n * es, 0, ((size_t)c.G.fsize - n) * es);
+    return hipMemsetAsync((char *)c.w.heating_diss.p + n * es, 0, ((size_t)c.G.fsize - n) * es, h->stream);
   };
-  if (h->c.C.lklemp) HIPCHK(h, h->mixed ? zero_below(h->cf) : zero_below(h->c));
+  if (h->c.C.lklemp) {  // on the handle's stream, which does not wait for the null stream
+    HIPCHK(h, h->mixed ? zero_below(h->cf) : zero_below(h->c));
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+  }
   h->rad_calls = hd.rad_calls;
   return LGAME_OK;
 }

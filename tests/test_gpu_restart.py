@@ -16,6 +16,7 @@ from lgame import surrogate
 from lgame.cases import make_case, moist3d_config, radiation_surface, schaer_config, tiny_config
 from lgame.config import PREC_FP64, PREC_MIXED, RAD_SURROGATE, RAD_TEACHER
 from lgame.gpu import LgameError, Step
+from pyoracle import CpuOracle
 
 pytestmark = pytest.mark.gpu
 T0 = surrogate.T_EPOCH + 3 * 3600.0
@@ -180,3 +181,26 @@ def test_diagnosing_a_slot_keeps_the_carried_fields(precision):
     assert b.checkpoint() == blob
     a.close()
     b.close()
+
+
+def test_restored_dissipation_rate_is_zero_below_the_klemp_layer():
+    """With the Klemp layer as the only dissipation the rate is formed in its levels: a checkpoint that holds
+    other values below them leaves zeros there, as soon as it is loaded, and the rate in the levels above."""
+    cfg, g, st, _, _ = _restart_case("dry")
+    a = Step(cfg, g)
+    a.start(st)
+    a.run(0, 5)
+    rate, blob = a.diag("heating_diss"), bytearray(a.checkpoint())
+    levels = CpuOracle(cfg, g).n_damping_levels
+    assert 0 < levels < cfg.n_layers and np.abs(rate).max() > 0.0
+    pitch = (cfg.nx + 1 + 15) // 16 * 16
+    shape = (cfg.n_layers + 1, cfg.ny + 1, pitch)
+    offset = 56 + 19 * 8 * int(np.prod(shape))  # after the header and 8 boxes of the pressure gradient, 10 of the advection and 1 of the sediment heating
+    box = np.frombuffer(blob, dtype=np.float64, count=int(np.prod(shape)), offset=offset).reshape(shape).copy()
+    assert np.array_equal(box[:cfg.n_layers, :cfg.ny, :cfg.nx].transpose(1, 2, 0), rate)
+    box[levels:] = 1.0
+    blob[offset:offset + box.nbytes] = box.tobytes()
+    for _ in range(3):
+        a.restore(bytes(blob))
+        assert np.array_equal(a.diag("heating_diss"), rate)
+    a.close()
