@@ -1,13 +1,16 @@
 """Launch tuning and ensembles: the autotuner's block shapes, the vertical segments of the
-column-marching scalar kernel and the graph-captured ensemble step must not change any result
+column-marching kernels, the column solvers and the graph-captured ensemble step must not change any result
 (every member stays bitwise equal to its own oracle run)."""
 import dataclasses
 
 import numpy as np
 import pytest
 
+from golden_util import max_rel
 from lgame.cases import dry3d_config, make_case, tiny_config
+from lgame.config import PREC_FP64, PREC_MIXED
 from lgame.gpu import TILE_KERNELS, Ensemble, LgameError, Step
+from lgame.metrics import field_errors, worst
 from pyoracle import CpuOracle
 
 pytestmark = pytest.mark.gpu
@@ -75,8 +78,8 @@ VER_CASES = {
 
 @pytest.mark.parametrize("name", list(VER_CASES))
 def test_vertical_solver_passes_keep_results(name):
-    """The vertical solver in one pass per column and in three passes (rows, Thomas recursion,
-    new state), each bitwise equal to the oracle; small domains default to three passes."""
+    """The setting of the vertical solver's passes, which columns of up to 72 layers keep and do not
+    use: bitwise equal to the oracle with either; small domains default to three passes."""
     cfg, n, cf = VER_CASES[name]
     g, st = make_case(cfg, cloud_frac=cf)
     want = _oracle(cfg, g, st, n)
@@ -95,6 +98,61 @@ def test_vertical_solver_passes_keep_results(name):
     with pytest.raises(LgameError, match="passes"):
         s.column_passes = 2
     s.close()
+
+
+TALL_CASES = {
+    "dry_o2": (tiny_config(ny=6, nx=70, n_layers=73), 4, 0.0),
+    "dry_o3_freeslip_diff": (tiny_config(ny=5, nx=33, n_layers=80, order=3, freeslip=True).set_diffusion(True), 4, 0.0),
+    # five column wavefronts (an odd one for the tracer solver's pairs), and two to a row
+    "moist_o3_freeslip": (tiny_config(ny=5, nx=11, n_layers=74, moist=True, order=3, freeslip=True), 5, 0.3),
+    "moist_two_wavefronts": (tiny_config(ny=3, nx=65, n_layers=73, moist=True), 4, 0.3),
+    "diff_pbl_soil_sens": (dataclasses.replace(tiny_config(ny=5, nx=9, n_layers=79, moist=True, order=3).set_diffusion(True),
+                                               lpbl=True, lprog_soil_temp=True, lsfc_sensible_heat_flux=True), 6, 0.3),
+}
+
+
+@pytest.mark.parametrize("precision", [PREC_FP64, PREC_MIXED])
+@pytest.mark.parametrize("name", list(TALL_CASES))
+def test_tall_column_solvers_match_oracle(name, precision):
+    """Columns of more than 72 layers, which the solvers in registers do not take: the vertical solver in
+    one pass per column and in three (rows, Thomas recursion, new state), the tracer solver through the
+    column scratch.  Both passes give the same bits.  Against the oracle the dry FP64 form is bitwise,
+    the others agree to rounding (the device's exp, log and pow); the mixed form has its own bar."""
+    cfg, n, cf = TALL_CASES[name]
+    g, st = make_case(cfg, cloud_frac=cf)
+    want = _oracle(cfg, g, st, n)
+    got = {}
+    for passes in (1, 3):
+        s = Step(dataclasses.replace(cfg, precision=precision), g)
+        s.column_passes = passes
+        s.start(st)
+        s.run(0, n)
+        got[passes] = s.get_state(n % 2)
+        s.close()
+        print(f"{name}: passes {passes}", flush=True)
+    assert all(np.array_equal(got[1][k], got[3][k]) for k in want)
+    if precision == PREC_MIXED:
+        err = field_errors(got[1], want)
+        assert worst(err, "rms_rel") < 1e-4 and worst(err, "max_rel") < 1e-4
+    elif cfg.lmoist:
+        assert max_rel(got[1], want) <= 1e-12
+    else:
+        assert all(np.array_equal(got[1][k], want[k]) for k in want)
+
+
+def test_autotune_of_tall_columns_keeps_results():
+    """The autotuner also times the vertical solver's passes where columns use them."""
+    cfg, n, _ = TALL_CASES["dry_o2"]
+    g, st = make_case(cfg)
+    s = Step(cfg, g)
+    s.start(st)
+    s.autotune(2)
+    assert s.column_passes in (1, 3)
+    s.run(0, n)
+    got = s.get_state(n % 2)
+    s.close()
+    want = _oracle(cfg, g, st, n)
+    assert all(np.array_equal(got[k], want[k]) for k in want)
 
 
 @pytest.mark.parametrize("nl,nx,moist", [(3, 4, False), (7, 31, False), (8, 32, True), (9, 33, False), (40, 65, False), (41, 5, True),
@@ -191,6 +249,53 @@ def test_tracer_solver_levels_match_oracle(nl, nx):
     got = s.get_state(1)
     s.close()
     assert all(np.array_equal(got[k], want[k]) for k in want)
+
+
+@pytest.mark.parametrize("precision,nx", [(PREC_FP64, 9), (PREC_FP64, 64), (PREC_FP64, 70), (PREC_MIXED, 70)])
+def test_lowest_tall_tracer_columns_match_oracle(precision, nx):
+    """65 layers, the first height of the tracer solver's tall form.  At nx 70 the FP64 form differs from the
+    oracle by one unit in the last place of wind_w and cloud water in one column, where the device's exp in the
+    heat capacity of ice is one unit from the host's: agreement to rounding, and the mixed form's own bar."""
+    cfg = dataclasses.replace(tiny_config(ny=3, nx=nx, n_layers=65, moist=True), n_oro_layers=61)
+    g, st = make_case(cfg, cloud_frac=0.3)
+    want = _oracle(cfg, g, st, 3)
+    s = Step(dataclasses.replace(cfg, precision=precision), g)
+    s.start(st)
+    s.run(0, 3)
+    got = s.get_state(1)
+    s.close()
+    if precision == PREC_MIXED:
+        err = field_errors(got, want)
+        assert worst(err, "rms_rel") < 1e-4 and worst(err, "max_rel") < 1e-4
+    else:
+        assert max_rel(got, want) <= 1e-12
+
+
+@pytest.mark.parametrize("layers", [(40, 64, 65, 72), (40, 65, 72, 73)])
+def test_batched_mixed_members_of_different_height_match_single(layers):
+    """The mixed form of a batched group whose members take different column solvers: every member has
+    the bits it has when stepped alone."""
+    cfgs = [dataclasses.replace(tiny_config(ny=4, nx=20 + 25 * i, n_layers=nl, moist=True), precision=PREC_MIXED)
+            for i, nl in enumerate(layers)]
+    cases = [make_case(c, cloud_frac=0.3) for c in cfgs]
+    steps = []
+    for c, (g, st) in zip(cfgs, cases):
+        s = Step(c, g)
+        s.start(st)
+        steps.append(s)
+    e = Ensemble(steps)
+    e.run(0, 3, mode=Ensemble.BATCHED)
+    e.sync()
+    for c, (g, st), s in zip(cfgs, cases, steps):
+        one = Step(c, g)
+        one.start(st)
+        one.run(0, 3)
+        got, want = s.get_state(1), one.get_state(1)
+        one.close()
+        assert all(np.array_equal(got[k], want[k]) for k in want), c.n_layers
+    e.close()
+    for s in steps:
+        s.close()
 
 
 def test_batched_tracer_solver_with_members_of_different_height():
