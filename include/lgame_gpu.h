@@ -474,7 +474,8 @@ int lgame_profile_reset(lgame_handle *h);
  * The scalar divergence, theta_div and diff_flux kernels march down the columns; their levels can
  * be cut into 1, 2, 4 or 8 segments (at least 4 levels each) so that small domains fill the GPU:
  * lgame_init picks the segments that give about four wavefronts per SIMD,
- * lgame_autotune times 1, 2, 4 and 8 after the block shapes, lgame_set_segments sets them and
+ * lgame_autotune times 1, 2, 4 and 8 after the block shapes and keeps the smallest sum of these
+ * kernels' times, lgame_set_segments sets them and
  * lgame_get_segments reads the choice.  Every choice gives the same bits. */
 #define LGAME_N_TILES 21
 int lgame_autotune(lgame_handle *h, int steps, int *rows);

@@ -57,7 +57,7 @@ struct MemberDev {
   StateDev s[2];
   RadDev rad;
   double t_rad;
-  int seg;  // vertical segments of the column-marching scalar kernel
+  int seg;  // vertical segments of the column-marching kernels
 };
 
 // the arguments that are the same for every member of a launch

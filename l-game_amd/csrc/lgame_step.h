@@ -48,7 +48,7 @@ enum KernelId {
 };
 
 // rows per block of every stencil kernel (block = 64 x by threads), and the number of vertical
-// segments of the column-marching scalar kernel
+// segments of the column-marching kernels
 struct Tiles {
   int by[KI_COUNT];
   int seg = 1;

@@ -295,7 +295,7 @@ class Step:
 
     @property
     def segments(self) -> int:
-        """Vertical segments of the column-marching scalar kernel."""
+        """Vertical segments of the column-marching kernels."""
         n = ctypes.c_int(0)
         self._check(self.lib.lgame_get_segments(self.h, ctypes.byref(n)), "lgame_get_segments")
         return n.value

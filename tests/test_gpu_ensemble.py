@@ -9,7 +9,7 @@ import pytest
 from golden_util import max_rel
 from lgame.cases import dry3d_config, make_case, tiny_config
 from lgame.config import PREC_FP64, PREC_MIXED
-from lgame.gpu import TILE_KERNELS, Ensemble, LgameError, Step
+from lgame.gpu import TILE_KERNELS, Ensemble, LgameError, Step, grid_setup_device
 from lgame.metrics import field_errors, worst
 from pyoracle import CpuOracle
 
@@ -64,6 +64,19 @@ def test_scalar_kernel_segments_and_rows_keep_results():
     for bad in (3, 8):  # not a power of two; fewer than 4 levels per segment
         with pytest.raises(LgameError, match="segment"):
             s.segments = bad
+    s.close()
+
+
+def test_autotune_times_all_kernels_that_the_segments_cut():
+    """161x129x47 with third-order theta in FP64: the scalar kernel alone is fastest with 2 segments (82 us,
+    89 with 4), together with the theta kernel it is not (205 us, 191 with 4 and 196 with 8)."""
+    cfg = dataclasses.replace(dry3d_config(n=129, n_layers=47), ny=161, theta_adv_order=3)
+    g, st = make_case(cfg, grid=grid_setup_device(cfg))
+    s = Step(cfg, g)
+    s.start(st)
+    s.autotune(16)
+    print(f"segments {s.segments}", flush=True)
+    assert s.segments in (4, 8)
     s.close()
 
 
