@@ -295,8 +295,8 @@ __global__ void __launch_bounds__(BX * BY) k_diff_mom(const CtxT<R> c, const Sta
 // with 24 flux fields in between (moist) it moved 723 B per cell in FP64 where 264 are needed.
 // It is bound by its instructions now, one wavefront per SIMD in FP64 (380 registers, 12,900 cycles a
 // layer): eight quotients per field and cell, which share seven denominators, and no branches in the
-// field loop (with them 526 us in FP64).  Both kernels before -> this one, us: 256x256x60 FP64 759 -> 456,
-// 321x225x51 mixed 482 -> 248.
+// field loop (with them 526 us in FP64).  Both kernels before -> this one, us: 256x256x60 FP64 759 -> 445,
+// 321x225x51 mixed 482 -> 247.
 // ---------------------------------------------------------------------------------------------
 template <class R>
 __device__ __forceinline__ R c_g_v(R rg) {

@@ -28,10 +28,12 @@ __device__ __forceinline__ int wrapm(int i, int n) { return i == 1 ? n : i - 1; 
 // a - b*q is exact in one fused multiply-add, and a correction with y leaves less than one unit, after
 // which a second correction rounds as a/b does (P. Markstein, "Computation of elementary functions on
 // the IBM RISC System/6000 processor", IBM J. Res. Dev. 34, 1990).  Where the residual is not a number
-// (an infinite a or b), q itself is the operator's value.  (Below about 1e-290 the residual can
-// underflow and the last place may differ.)
+// (an infinite a or b), q itself is the operator's value.  Two exceptions, neither of which reaches a
+// result of the kernels that divide so: below about 1e-290 the residual can underflow and the last place
+// may differ, and -0/b gives +0 (the residual is +0 and is added).  b is not subnormal.
 // FP32: the FP64 product is off by at most 2^-51 relative, and a quotient of two 24-bit numbers is never
-// within 2^-49 of the middle between two 24-bit numbers, so its rounding is that of a/b.
+// within 2^-49 of the middle between two 24-bit numbers, so its rounding is that of a/b (where the
+// quotient is a normal number; a subnormal one has fewer bits and its last one may differ).
 // Five fused operations and a select (FP64) or a product between two conversions (FP32) take the place
 // of the operator's scaled Newton iteration of twelve, five of them at a quarter of the rate.
 template <class R>

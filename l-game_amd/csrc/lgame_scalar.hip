@@ -331,7 +331,7 @@ void launch_scalar_col(const CtxT<R> &c, const StateDev &ss, const StateDev &nw,
   const int tx_n = (c.G.nx + SCOL_CELLS - 1) / SCOL_CELLS, ty_n = (c.G.ny + rows - 1) / rows;
   const dim3 blk(BX, rows, 1), grd((unsigned)(tx_n * ty_n * nseg));
   const bool tr = c.G.nc > 1, o3 = c.C.order == 3, diff = scol_diff_variant<R>(c.C.ltemp_h || c.C.lmass_h);
-const bool told = tr && rk == 2;
+  const bool told = tr && rk == 2;
 #define LG_SCOL(TR, O3, DIFF, TOLD) hipLaunchKernelGGL((k_scalar_col<R, TR, O3, DIFF, TOLD>), grd, blk, 0, st, c, ss, nw, nseg)
   LG_SCOL_DISPATCH
 #undef LG_SCOL
@@ -348,8 +348,8 @@ template void launch_scalar_col<float>(const CtxT<float> &, const StateDev &, co
 // As a gradient kernel and a divergence kernel the gradients went through memory (four fields at the
 // first substep) and the metrics of three layers were loaded for every cell; both kernels were bound by
 // their load instructions.
-// FP64 161x129x47, us: the two kernels before 113 (mean of a step's two substeps) -> 48 (51 with two fields,
-// 45 with one); 201x3x40: 13.3 -> 12.4.
+// FP64 161x129x47 with 8 segments, us: the two kernels before 113 (mean of a step's two substeps) -> 46 (49 with
+// two fields, 44 with one); 201x3x40: 13.3 -> 11.5.
 // The gradients at column nx+1 and row ny+1 take the covariant part and the remap of column 1 and
 // row 1 and the slope stored there (grad_hor_x/_y).
 // NF: 2 fields, the full theta_v and its perturbation, or the first alone
@@ -502,7 +502,7 @@ template <class R>
 void batch_launch_scalar(dim3 g, dim3 b, hipStream_t st, const MemberDev<R> *M, const int *prefix, int nm, const BatchArgs &a,
                          bool tr, bool o3, bool diff) {
   diff = scol_diff_variant<R>(diff);
-const bool told = tr && a.rk == 2;
+  const bool told = tr && a.rk == 2;
 #define LG_SCOL(TR, O3, DIFF, TOLD) hipLaunchKernelGGL((kb_scalar_col<R, TR, O3, DIFF, TOLD>), g, b, 0, st, M, prefix, nm, a)
   LG_SCOL_DISPATCH
 #undef LG_SCOL

@@ -315,10 +315,11 @@ __global__ void __launch_bounds__(BCOL) k_solve_ver(const CtxT<R> c, const State
 // one lane per (column, segment).  All lanes load their layers and form their rows of the system at
 // once; then only the Thomas recursion runs from segment to segment (the lanes of one segment at a
 // time, the eliminated coefficients of its last row through LDS), down and back up; then all lanes
-// form the new state.  Between the phases a lane keeps its rows, the explicit densities, gamma and
-// theta_v at the interfaces in registers and the old state and volume of its layers in LDS, so the
-// column scratch and the second reads of most inputs of ver_column are gone.  The expressions are
-// those of ver_column, so the results are the same bits.
+// form the new state.  Between the phases a lane keeps its rows, gamma and theta_v at the interfaces in
+// registers and the old and the explicit densities of its layers in LDS, so the column scratch and the
+// second reads of most inputs of ver_column are gone (the volume, the old Exner pressure and w, the
+// background theta_v and the interface area are loaded once more, during the back substitution).  The
+// expressions are those of ver_column, so the results are the same bits.
 //
 // What bounds it: memory traffic and the divisions of the rows on large domains, the recursion's chain
 // of dependent divisions and the latency of one block on small ones.  A CU's registers and LDS hold 64
@@ -363,7 +364,9 @@ __device__ __forceinline__ void ver_segment(const CtxT<R> &c, const StateDev &ol
     if (ahead) nxt = load_raw(c, old, nu, RK, ix(l0 + 2));
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      if (ahead && k * VS_SEG >= nl) break;  // longer than this column's segments
+      // longer than this column's segments (K = 9 is for columns of over 64 layers, which use all of it; the
+      // shorter members of a batched group form rows there that they do not use)
+      if (ahead && k * VS_SEG >= nl) break;
       RawLayer cur;  // layer l0+k+2
       if (ahead) {
         cur = nxt;
@@ -1116,9 +1119,11 @@ __global__ void __launch_bounds__(BCOL * NTR * GEN_GROUPS) k_solve_gen(const Ctx
 // One barrier per KX levels: behind it the tracers read levels of the ring while the next KX are written,
 // and leave heating terms while those of the previous KX are added up.  KX is 4, or 2 with the heating, where
 // the ring holds more; half of that in columns of 65 to 72 layers (TALL), whose e' leaves less LDS.
-// Bound by memory traffic (the scratch was 160 of 350 B per tracer column and level): us per launch at the
-// predictor and the corrector, k_solve_gen -> here: 512x512x60 FP64 1240, 1030 -> 880, 718 (4.5 TB/s), mixed
-// 1190, 990 -> 851, 703; 257x193x55 FP64 240 (mean) -> 203, 162; tall, 291x209x69 mixed 428 (mean) -> 352, 255.
+// The scratch was 160 of 350 B per tracer column and level.  us per launch at the predictor and the corrector,
+// k_solve_gen -> here: 512x512x60 FP64 1240, 1030 -> 889, 725, mixed 1190, 990 -> 861, 697; 257x193x55 FP64 240
+// (mean) -> 205, 164; tall, 291x209x69 mixed 428 (mean) -> 352, 255.  It moves 3.6 and 4.1 TB/s (FP64) where a large
+// copy moves 5.1, with the address unit busy a third of the time: the one block of a CU only loads while it
+// eliminates and only stores while it substitutes.
 // Without the seventh wavefront (each tracer loading everything, two levels ahead) it was bound by latency:
 // 1517, 991.
 typedef double GenVec __attribute__((ext_vector_type(GR_PART)));

@@ -82,7 +82,7 @@ constexpr int BCOL = 64;
 // per block, segments per column.
 constexpr int VS_COLS = 32, VS_SEG = 8;
 constexpr int VS_THREADS = VS_COLS * VS_SEG;
-constexpr int VS_LDS = 4;   // arrays of a column kept in LDS: old rho, rhotheta_v, Exner pressure and the volume
+constexpr int VS_LDS = 4;   // arrays of a column kept in LDS: the old and the explicit rho and rhotheta_v
 constexpr int VS_XCH = 3 * VS_SEG + 1;  // doubles per column exchanged between segments
 // bytes of LDS a block needs for nl levels
 __host__ __device__ inline size_t vs_lds_bytes(int nl) { return sizeof(double) * VS_COLS * ((size_t)VS_LDS * nl + VS_XCH); }
