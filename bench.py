@@ -88,10 +88,10 @@ STEP_BYTES = {"dry": 920.0, "moist": 1296.0}  # per grid-point step, whole-step 
 SOLVER_TRAFFIC = {("moist512", "fp64"): 3.435e+09, ("moist512", "mixed"): 3.326e+09}
 # the same for the kernels of KERNEL_BYTES, (workload, kernel, form) -> bytes per launch
 KERNEL_TRAFFIC = {("moist512", "solve_ver", "fp64"): 3.435e+09, ("moist512", "solve_ver", "mixed"): 3.326e+09,
-                  ("moist512", "scalar_div", "fp64"): 5.900e+09, ("moist512", "scalar_div", "mixed"): 4.113e+09,
+                  ("moist512", "scalar_div", "fp64"): 5.865e+09, ("moist512", "scalar_div", "mixed"): 3.915e+09,
                   ("moist512", "solve_gen", "fp64"): 3.085e+09, ("moist512", "solve_gen", "mixed"): 2.750e+09}
 # measured HBM bytes per grid-point step of the whole FP64 step (same counters, all kernels)
-STEP_TRAFFIC = {"moist512": 2873.0}
+STEP_TRAFFIC = {"moist512": 2878.0}
 # the reference's own CPU path, flang -O2 -fopenmp on 8 cores, measured on an 8-core Xeon host (the
 # reference tree does not travel, so it cannot be timed beside the GPU)
 REFERENCE_CPU = {"dry128": {"value": 3.19e6, "grid": "129x129x50 dry", "cores": 8},
