@@ -300,7 +300,9 @@ int lgame_checkpoint_load(lgame_handle *h, const void *buf, long long bytes);
 #define LGAME_DIAG_MOM_DIFF_TEND_X 3   /* diag%mom_diff_tend_x (ny,nx+1,nl)                         */
 #define LGAME_DIAG_MOM_DIFF_TEND_Z 4   /* diag%mom_diff_tend_z (ny,nx,nl+1)                         */
 #define LGAME_DIAG_TEMP_DIFF_HEATING 5 /* diag%temp_diff_heating (ny,nx,nl)                         */
-#define LGAME_DIAG_HEATING_DISS    6   /* diag%heating_diss (ny,nx,nl)                              */
+#define LGAME_DIAG_HEATING_DISS    6   /* diag%heating_diss (ny,nx,nl); with the Klemp layer as the only
+                                        * dissipation it is formed in the layer's levels and zero in
+                                        * those below, whatever the wind there (it has a zero factor) */
 #define LGAME_DIAG_ROUGHNESS_LENGTH 7  /* diag%roughness_length (ny,nx), with the surface switches   */
 #define LGAME_DIAG_MONIN_OBUKHOV   8   /* diag%monin_obukhov_length (ny,nx), same                   */
 #define LGAME_DIAG_SCALAR_FLUX_RESISTANCE 9 /* diag%scalar_flux_resistance (ny,nx), with the sensible heat flux */
